@@ -337,15 +337,16 @@ int axf_hip_sample(axf_ctx* ctx, float* logits_dev, int n_vocab, const axf_sampl
     int* d_hist = reinterpret_cast<int*>(static_cast<uint8_t*>(scratch) + hist_off);
     int* d_hist_n = d_hist + n_hist;
     int* d_tok = d_hist_n + 1;
+    SamplePenalty pen;
     if (s->rep_penalty != 1.0f && n_hist > 0) {
         AXF_HIP(hipMemcpyAsync(d_hist, hist, (size_t)n_hist * 4, hipMemcpyHostToDevice,
                                ctx->stream));
         AXF_HIP(hipMemcpyAsync(d_hist_n, &n_hist, 4, hipMemcpyHostToDevice, ctx->stream));
-        AXF_HIP(launch_rep_penalty(logits_dev, d_hist, d_hist_n, s->rep_penalty_last_n,
-                                   s->rep_penalty, n_vocab, ctx->stream));
+        pen = {d_hist, d_hist_n, s->rep_penalty_last_n, s->rep_penalty};
     }
     AXF_HIP(launch_sample(d_tok, cand, logits_dev, n_vocab, s->temperature, s->top_k, s->top_p,
-                          nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr, ctx->stream));
+                          nullptr, r, nullptr, nullptr, nullptr, nullptr, nullptr, pen,
+                          ctx->stream));
     AXF_HIP(hipMemcpyAsync(token, d_tok, 4, hipMemcpyDeviceToHost, ctx->stream));
     AXF_HIP(hipStreamSynchronize(ctx->stream));
     return AXF_OK;

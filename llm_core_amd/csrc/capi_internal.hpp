@@ -299,12 +299,18 @@ hipError_t launch_push_token(int* tokens, int* step, const int* tok, hipStream_t
 // candidate keys (uint64) launch_sample needs in `cand`, 0 when k is beyond
 // the device path.
 int sample_candidates(int n_vocab, int k);
-hipError_t launch_rep_penalty(float* logits, const int* hist, const int* hist_n, int last_n,
-                              float penalty, int n_vocab, hipStream_t st);
-hipError_t launch_sample(int* out, uint64_t* cand, const float* logits, int n_vocab,
+// The repetition penalty that comes first (in place on the logits): the last
+// last_n of hist[0 .. *hist_n); none when hist_n is nullptr.
+struct SamplePenalty {
+    const int* hist = nullptr;
+    const int* hist_n = nullptr;
+    int last_n = 0;
+    float penalty = 1.f;
+};
+hipError_t launch_sample(int* out, uint64_t* cand, float* logits, int n_vocab,
                          float temperature, int top_k, float top_p, const float* r_table,
                          float r_fixed, int* tokens, int* step, int* pos, int* hist, int* hist_n,
-                         hipStream_t st);
+                         const SamplePenalty& pen, hipStream_t st);
 void sampling_uniforms(uint32_t seed, float* out, int n);
 // effective k of sample() (llama_model.cpp:1473): 1 for greedy
 inline int sample_k(const axf_sampling& s, int n_vocab) {

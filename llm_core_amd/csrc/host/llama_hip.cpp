@@ -610,15 +610,13 @@ hipError_t enqueue_pick(axf_llama* m, bool record, bool advance_pos, const axf_s
         return launch_argmax(m->d_token, m->arg_v, m->arg_i, m->logits, hp.n_vocab,
                              record ? m->d_tokens : nullptr, record ? m->d_step : nullptr,
                              advance_pos ? m->d_pos : nullptr, st);
-    if (smp->rep_penalty != 1.0f) {
-        hipError_t e = launch_rep_penalty(m->logits, m->d_hist, m->d_hist_n,
-                                          smp->rep_penalty_last_n, smp->rep_penalty, hp.n_vocab, st);
-        if (e != hipSuccess) return e;
-    }
+    SamplePenalty pen;
+    if (smp->rep_penalty != 1.0f)
+        pen = {m->d_hist, m->d_hist_n, smp->rep_penalty_last_n, smp->rep_penalty};
     return launch_sample(m->d_token, m->d_cand, m->logits, hp.n_vocab, smp->temperature,
                          smp->top_k, smp->top_p, m->d_r, 0.f, record ? m->d_tokens : nullptr,
                          record ? m->d_step : nullptr, advance_pos ? m->d_pos : nullptr,
-                         m->d_hist, m->d_hist_n, st);
+                         m->d_hist, m->d_hist_n, pen, st);
 }
 
 // The step's head: logits and the greedy pick (the fused argmax where it applies).

@@ -22,6 +22,9 @@
 //      the host from the reference's std::mt19937 stream.
 // Greedy (temperature <= 0) is the same path with k = 1 on the raw logits:
 // the first index of the maximum, std::max_element.
+// Up to 64 candidates (the default top_k is 40) nothing is sorted: steps 1 and
+// 2 are k_topk_select and step 3 is k_sample_pick_select, which find the k
+// best by a threshold and rank them (below); the same tokens and logits.
 #include "common.hpp"
 
 namespace axf {
@@ -109,10 +112,24 @@ __device__ void pick_sorted(uint64_t* keys, const uint64_t* __restrict__ cand, i
     bitonic_desc<N>(keys);
 }
 
-// Final choice over keys sorted in descending order (one thread).  Outputs as
-// the greedy argmax kernel: *out, and when given tokens[*step] = token,
-// *step += 1, *pos += 1; the token is always appended to the penalty history
-// (hist[*hist_n], *hist_n += 1) when hist is given.
+// Outputs as the greedy argmax kernel: *out, and when given tokens[*step] =
+// token, *step += 1, *pos += 1; the token is always appended to the penalty
+// history (hist[*hist_n], *hist_n += 1) when hist is given.
+__device__ __forceinline__ void record_pick(int chosen, int* out, int* tokens, int* step, int* pos,
+                                            int* hist, int* hist_n) {
+    *out = chosen;
+    if (tokens && step) {
+        tokens[*step] = chosen;
+        *step += 1;
+    }
+    if (pos) *pos += 1;
+    if (hist && hist_n) {
+        hist[*hist_n] = chosen;
+        *hist_n += 1;
+    }
+}
+
+// Final choice over keys sorted in descending order (one thread).
 __device__ void finish_pick(const uint64_t* keys, int k, float top_p,
                             const float* __restrict__ r_table, float r_fixed, int* out,
                             int* tokens, int* step, int* pos, int* hist, int* hist_n) {
@@ -157,16 +174,7 @@ __device__ void finish_pick(const uint64_t* keys, int k, float top_p,
             }
         }
     }
-    *out = chosen;
-    if (tokens && step) {
-        tokens[*step] = chosen;
-        *step += 1;
-    }
-    if (pos) *pos += 1;
-    if (hist && hist_n) {
-        hist[*hist_n] = chosen;
-        *hist_n += 1;
-    }
+    record_pick(chosen, out, tokens, step, pos, hist, hist_n);
 }
 
 __global__ __launch_bounds__(kSortThreads) void k_sample_pick(
@@ -215,6 +223,213 @@ __global__ __launch_bounds__(kSortThreads) void k_sample_pick_large(
         finish_pick(cand, k, top_p, r_table, r_fixed, out, tokens, step, pos, hist, hist_n);
 }
 
+// ---------------------------------------------------------------------------
+// k <= 64 without a sort.  The k-th largest of a workgroup's per-thread maxima
+// is a lower bound of its k-th largest key, and (keys are distinct) only k
+// threads hold keys at or above it: at most k * (keys per thread) survive, k +
+// a few in practice, and a survivor's place is the number of survivors above
+// it.  The sorts these replace are ~78 barrier-separated LDS passes each and
+// one thread's chain of 3k expf; the bound here is the 256-way count over the
+// maxima (one pass over 2 KiB of LDS per thread) and the load latency.
+// 151936 logits, k = 40, 64 penalised ids: penalty + chunks + pick
+// 21.4 + 50.6 + 31.6 us with the walk and the sorts, 10.8 + 10.2 us here.
+// ---------------------------------------------------------------------------
+constexpr int kSelK = 64;         // largest k of this path
+constexpr int kSelThreads = 256;
+constexpr int kSelWindow = 1024;  // longest penalty window it takes
+
+template <int LIST>
+struct SelectShared {
+    uint64_t mx[kSelThreads];
+    uint64_t list[LIST];
+    unsigned long long thr;
+    int n;
+};
+
+// sh.thr = the k-th largest of the threads' own maxima (0 when fewer than k
+// are nonzero); sh.n = 0.  Every thread.
+template <int LIST>
+__device__ __forceinline__ void select_threshold(SelectShared<LIST>& sh, uint64_t mine, int k) {
+    sh.mx[threadIdx.x] = mine;
+    if (threadIdx.x == 0) {
+        sh.thr = ~0ull;
+        sh.n = 0;
+    }
+    __syncthreads();
+    int above = 0;
+#pragma unroll 16
+    for (int j = 0; j < kSelThreads; j++) above += sh.mx[j] > mine ? 1 : 0;
+    if (above < k) atomicMin(&sh.thr, (unsigned long long)mine);
+    __syncthreads();
+}
+
+template <int LIST>
+__device__ __forceinline__ void select_keep(SelectShared<LIST>& sh, uint64_t key, uint64_t thr) {
+    if (key != 0 && key >= thr) {
+        const int at = atomicAdd(&sh.n, 1);
+        if (at < LIST) sh.list[at] = key;
+    }
+}
+
+// out[r] = the key of rank r < k among the list's n, zeros past n
+template <int LIST>
+__device__ __forceinline__ void select_rank(const SelectShared<LIST>& sh, int k,
+                                            uint64_t* __restrict__ out) {
+    const int n = min(sh.n, LIST);
+    for (int i = threadIdx.x; i < n; i += kSelThreads) {
+        const uint64_t key = sh.list[i];
+        int above = 0;
+#pragma unroll 8
+        for (int j = 0; j < n; j++) above += sh.list[j] > key ? 1 : 0;
+        if (above < k) out[above] = key;
+    }
+    for (int i = n + (int)threadIdx.x; i < k; i += kSelThreads) out[i] = 0;
+}
+
+// A chunk of 4096 logits: the penalty of the ids in it (hist_n != nullptr;
+// an id seen m times is penalised m times, as k_rep_penalty's walk does), then
+// its k best keys in descending order.
+__global__ __launch_bounds__(kSelThreads) void k_topk_select(
+    uint64_t* __restrict__ cand, float* logits, int n_vocab, float temperature, int divide, int k,
+    const int* __restrict__ hist, const int* __restrict__ hist_n, int last_n, float penalty) {
+    constexpr int PER = kChunk / kSelThreads;
+    __shared__ SelectShared<kSelK * PER> sh;
+    __shared__ int stale[kSelThreads];  // the thread's logits hold a penalised one
+    const int base = blockIdx.x * kChunk, lim = min(base + kChunk, n_vocab);
+    // issued first: the penalty's chain of loads runs while they arrive
+    float x[PER];
+    auto load = [&] {
+#pragma unroll
+        for (int p = 0; p < PER; p++)
+            x[p] = logits[min(base + p * kSelThreads + (int)threadIdx.x, n_vocab - 1)];
+    };
+    load();
+    if (hist_n) {
+        int* ids = reinterpret_cast<int*>(sh.list);
+        static_assert(sizeof(sh.list) >= kSelWindow * sizeof(int), "penalty window");
+        const int n = *hist_n;
+        const int win = max(0, min(min(last_n, n), kSelWindow));
+        for (int i = threadIdx.x; i < win; i += kSelThreads) ids[i] = hist[n - win + i];
+        stale[threadIdx.x] = 0;
+        __syncthreads();
+        for (int i = threadIdx.x; i < win; i += kSelThreads) {
+            const int id = ids[i];
+            if (id < base || id >= lim) continue;
+            int times = 0, before = 0;
+            for (int j = 0; j < win; j++) {
+                times += ids[j] == id ? 1 : 0;
+                before += ids[j] == id && j < i ? 1 : 0;
+            }
+            if (before) continue;  // its first occurrence applies them all
+            float v = logits[id];
+            for (int j = 0; j < times; j++) v = v > 0.f ? v / penalty : v * penalty;
+            logits[id] = v;
+            stale[(id - base) % kSelThreads] = 1;
+        }
+        __syncthreads();
+        if (stale[threadIdx.x]) load();
+    }
+    uint64_t key[PER];
+    uint64_t mine = 0;
+#pragma unroll
+    for (int p = 0; p < PER; p++) {
+        const int i = base + p * kSelThreads + (int)threadIdx.x;
+        // 0 is below every real key
+        key[p] = i < n_vocab ? make_key(divide ? x[p] / temperature : x[p], i) : 0;
+        mine = key[p] > mine ? key[p] : mine;
+    }
+    select_threshold(sh, mine, k);
+    const uint64_t thr = sh.thr;
+#pragma unroll
+    for (int p = 0; p < PER; p++) select_keep(sh, key[p], thr);
+    __syncthreads();
+    select_rank(sh, k, cand + (size_t)blockIdx.x * k);
+}
+
+// finish_pick's choice by one wave, lane i holding key i: the exponentials and
+// divisions side by side, the sums in finish_pick's order (its second sum is
+// the running sum at the cut, so it is not repeated).
+__device__ __forceinline__ int wave_pick(uint64_t key, int k, float top_p, float r) {
+    const int lane = threadIdx.x & 63;
+    const int idx = (int)~(uint32_t)key;
+    if (k == 1) return __builtin_amdgcn_readlane(idx, 0);
+    auto bcast = [](float v, int i) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+    };
+    const float s = from_ordered((uint32_t)(key >> 32));
+    // lanes from k on add zeros, which change no sum: the loops unroll whole
+    const float e = lane < k ? expf(s - bcast(s, 0)) : 0.f;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < kSelK; i++) sum += bcast(e, i);
+    float p = e / sum;
+    // the running sums of p over 0..lane
+    auto running = [&] {
+        float cum = 0.f, own = 0.f;
+#pragma unroll
+        for (int i = 0; i < kSelK; i++) {
+            cum += bcast(p, i);
+            own = lane == i ? cum : own;
+        }
+        return own;
+    };
+    int kk = k;
+    if (top_p < 1.0f) {
+        const float own = running();
+        const uint64_t hit = __ballot(lane < k && own >= top_p);
+        kk = hit ? __builtin_ctzll(hit) + 1 : k;
+        p = p / bcast(own, kk - 1);
+    }
+    const float own = running();
+    const uint64_t hit = __ballot(lane < kk && r < own);
+    return __builtin_amdgcn_readlane(idx, hit ? __builtin_ctzll(hit) : kk - 1);
+}
+
+// The chunks' n_cand candidates (at most kPickMax) -> the step's token.
+__global__ __launch_bounds__(kSelThreads) void k_sample_pick_select(
+    int* __restrict__ out, const uint64_t* __restrict__ cand, int n_cand, int k, float top_p,
+    const float* __restrict__ r_table, float r_fixed, int* tokens, int* step, int* pos, int* hist,
+    int* hist_n) {
+    __shared__ SelectShared<kSelK * (kPickMax / kSelThreads)> sh;
+    __shared__ uint64_t best[kSelK];
+    // 8 candidates a thread in flight; up to 2048 of them stay in registers
+    constexpr int PER = 8;
+    uint64_t key[PER];
+    auto load = [&](int from) {
+#pragma unroll
+        for (int p = 0; p < PER; p++) {
+            const int i = from + p * kSelThreads + (int)threadIdx.x;
+            const uint64_t v = cand[min(i, n_cand - 1)];
+            key[p] = i < n_cand ? v : 0;
+        }
+    };
+    uint64_t mine = 0;
+    for (int from = 0; from < n_cand; from += PER * kSelThreads) {
+        load(from);
+#pragma unroll
+        for (int p = 0; p < PER; p++) mine = key[p] > mine ? key[p] : mine;
+    }
+    const float r = r_table ? r_table[step ? *step : 0] : r_fixed;
+    select_threshold(sh, mine, k);
+    const uint64_t thr = sh.thr;
+    for (int from = 0; from < n_cand; from += PER * kSelThreads) {
+        if (n_cand > PER * kSelThreads) load(from);
+#pragma unroll
+        for (int p = 0; p < PER; p++) select_keep(sh, key[p], thr);
+    }
+    __syncthreads();
+    select_rank(sh, k, best);
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int chosen = wave_pick(best[min((int)threadIdx.x, k - 1)], k, top_p, r);
+    if (threadIdx.x == 0) record_pick(chosen, out, tokens, step, pos, hist, hist_n);
+}
+
+// the select path's range: k, and the penalty window where there is one
+bool select_applies(int k, long n_cand, bool penalised, int last_n) {
+    return k <= kSelK && n_cand <= kPickMax && (!penalised || last_n <= kSelWindow);
+}
+
 }  // namespace
 
 int sample_chunks(int n_vocab) { return (n_vocab + kChunk - 1) / kChunk; }
@@ -235,23 +450,28 @@ int sample_candidates(int n_vocab, int k) {
     return p <= (1L << 30) ? (int)p : 0;
 }
 
-hipError_t launch_rep_penalty(float* logits, const int* hist, const int* hist_n, int last_n,
-                              float penalty, int n_vocab, hipStream_t st) {
-    hipLaunchKernelGGL(k_rep_penalty, dim3(1), dim3(1), 0, st, logits, hist, hist_n, last_n,
-                       penalty, n_vocab);
-    return hipGetLastError();
-}
-
-hipError_t launch_sample(int* out, uint64_t* cand, const float* logits, int n_vocab,
+hipError_t launch_sample(int* out, uint64_t* cand, float* logits, int n_vocab,
                          float temperature, int top_k, float top_p, const float* r_table,
                          float r_fixed, int* tokens, int* step, int* pos, int* hist, int* hist_n,
-                         hipStream_t st) {
+                         const SamplePenalty& pen, hipStream_t st) {
     const bool greedy = !(temperature > 0.f);
     int k = greedy ? 1 : ((top_k > 0 && top_k < n_vocab) ? top_k : n_vocab);
     const int kc = k < kChunk ? k : kChunk;
     const int chunks = sample_chunks(n_vocab);
     const int n_cand = (int)sample_n_cand(n_vocab, k);
     if (sample_candidates(n_vocab, k) == 0) return hipErrorInvalidValue;
+    if (select_applies(k, n_cand, pen.hist_n != nullptr, pen.last_n)) {
+        hipLaunchKernelGGL(k_topk_select, dim3(chunks), dim3(kSelThreads), 0, st, cand, logits,
+                           n_vocab, temperature, greedy ? 0 : 1, k, pen.hist, pen.hist_n,
+                           pen.last_n, pen.penalty);
+        hipLaunchKernelGGL(k_sample_pick_select, dim3(1), dim3(kSelThreads), 0, st, out, cand,
+                           n_cand, k, greedy ? 1.0f : top_p, r_table, r_fixed, tokens, step, pos,
+                           hist, hist_n);
+        return hipGetLastError();
+    }
+    if (pen.hist_n)
+        hipLaunchKernelGGL(k_rep_penalty, dim3(1), dim3(1), 0, st, logits, pen.hist, pen.hist_n,
+                           pen.last_n, pen.penalty, n_vocab);
     int pow2 = 1024;
     while (pow2 < n_cand) pow2 <<= 1;
     hipLaunchKernelGGL(k_topk_chunks, dim3(chunks), dim3(kSortThreads), 0, st, cand, logits,
