@@ -641,11 +641,15 @@ __global__ __launch_bounds__(256) void k_attn_prefill(AttnArgs a, int G, int QT)
 // merged at the end in wave order through LDS.  Per tile, straight from the
 // cache into registers (no LDS staging):
 //   S^T = K Q^T   v_mfma_f32_16x16x4_f32, A = 16 keys (lane: key col, dims
-//                 grp*HD/4 .. +HD/4, contiguous), B = the 16 query rows (same
-//                 dims); result lane: keys 4*grp + r of query col;
-//   O^T += V^T P^T  A = V (lane: keys 4*grp + r, dims col*HD/16 .. +HD/16),
+//                 16u + 4*grp .. +3 at HD 128), B = the 16 query rows (same dims);
+//                 result lane: keys 4*grp + r of query col;
+//   O^T += V^T P^T  A = V (lane: keys 4*grp + r, dims 64u + 4*col .. +3),
 //                 B = P as the S^T result lane holds it (no transpose);
-//                 result lane: dims (4*grp + r)*HD/16 + dt of query col.
+//                 result lane: dims 64u + 16*grp + 4*r .. +3 of query col.
+// The lanes of one load cover 64 contiguous bytes of each K row and 256 of each
+// V row: with a lane's dims contiguous instead, a K load touched 64 cache lines
+// for 16 bytes each, and 32 heads x 512 tokens at
+// position 1536 took 304 us instead of 183.
 // So the max over a tile's 16 keys is 4 values in the lane and two shuffles;
 // l stays per lane until the merge.  Four times the workgroups of the 64-row
 // kernel, longest key ranges first.  fp32 throughout; results differ from the
@@ -655,17 +659,67 @@ constexpr int kPfKsRows = 16;
 constexpr int kPfKsWaves = 4;
 
 template <int HD>
-__global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a, int G, int QT) {
+struct PrefillKsShared {
+    static constexpr int QS = HD + 4;  // LDS row stride (Q tile, then the waves' O rows)
+    __attribute__((aligned(16))) float qs[kPfKsWaves * kPfKsRows * QS];
+    float mm[kPfKsWaves][kPfKsRows], ll[kPfKsWaves][kPfKsRows];
+};
+
+// Four output values (dims 4*c4 ..) of query head `head` of token t: the fp32
+// row, its Q8_0 block with outq8 (8 consecutive lanes hold a block) and, with
+// xh, the block's re-layout for the o projection.
+template <int HD>
+__device__ __forceinline__ void store_out4(const AttnArgs& a, int t, int head, int c4, float4 v) {
+    const size_t e0 = (size_t)t * a.out_ld + (size_t)head * HD + 4 * c4;
+    float* dst = a.out + e0;
+    dst[0] = v.x;
+    dst[1] = v.y;
+    dst[2] = v.z;
+    dst[3] = v.w;
+    if (a.outq8) {
+        const int sub = c4 & 7;
+        float d;
+        const uint32_t p = q8_quant4(v, d);  // q8_store4's block
+        uint8_t* blk = a.outq8 + (e0 >> 5) * Q8_0_BYTES;
+        *reinterpret_cast<uint32_t*>(blk + 4 + 4 * sub) = p;
+        if (sub == 0) *reinterpret_cast<float*>(blk) = d;
+        if (a.xh) {  // k_gemm_prep16's re-layout of the block (out_ld % 32 == 0)
+            const int kb = (int)((e0 - (size_t)t * a.out_ld) >> 5), Tp = a.Tp;
+            _Float16 hv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) hv[e] = (_Float16)(float)(int8_t)(p >> (8 * e));
+            *reinterpret_cast<uint2*>(a.xh + (((size_t)kb * 4 + (sub >> 1)) * Tp + t) * 16 +
+                                      (sub & 1) * 8) = *reinterpret_cast<const uint2*>(hv);
+            int sum = dot4((int)p, 0x01010101, 0);
+            sum += __shfl_xor(sum, 1, 8);
+            sum += __shfl_xor(sum, 2, 8);
+            sum += __shfl_xor(sum, 4, 8);
+            if (sub == 0) {
+                const size_t i2 = (((size_t)kb * (Tp / 32) + t / 32) * 16 + (t & 15)) * 2 + ((t >> 4) & 1);
+                const size_t i4 = (((size_t)kb * (Tp / 64) + t / 64) * 16 + (t & 15)) * 4 + ((t >> 4) & 3);
+                a.dx2[i2] = d;
+                a.gx2[i2] = d * (float)sum;
+                a.dx4[i4] = d;
+            }
+        }
+    }
+}
+
+// 16 query rows (tokens qt0 .. qt0 + QT - 1) of kv head kvh, one workgroup.
+template <int HD, bool PF>
+__device__ __forceinline__ void prefill_rows16(const AttnArgs& a, int G, int QT, int kvh, int qt0,
+                                               PrefillKsShared<HD>& sh) {
     constexpr int KQ = HD / 4;   // dims per lane group: the k-steps of S^T
     constexpr int DT = HD / 16;  // dims per lane of a V row: the output tiles
+    // a lane's K dims: float4s KU floats apart from KL * grp on (64-dim rows are
+    // one cache line pair either way, and contiguous lanes were 2% faster there)
+    constexpr int KU = HD == 64 ? 4 : 16, KL = HD == 64 ? KQ : 4;
     constexpr int HALF = HD / 2;
-    constexpr int QS = HD + 4;   // LDS row stride (Q tile, then the waves' O rows)
+    constexpr int QS = PrefillKsShared<HD>::QS;
     constexpr int R = kPfKsRows, NW = kPfKsWaves;
-    __shared__ __attribute__((aligned(16))) float qs[NW * R * QS];
-    __shared__ float mm[NW][R], ll[NW][R];
-
-    const int kvh = blockIdx.x;
-    const int qt0 = (int)(gridDim.y - 1 - blockIdx.y) * QT;  // longest key ranges first
+    float* qs = sh.qs;
+    auto& mm = sh.mm;
+    auto& ll = sh.ll;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, grp = lane >> 4;
@@ -701,10 +755,10 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
         }
         __syncthreads();
     }
-    float qb[KQ];  // B operand of S^T: query col, dims grp*KQ + s
+    float qb[KQ];  // B operand of S^T: query col, dims KU*u + KL*grp + (s & 3), u = s / 4
 #pragma unroll
     for (int u = 0; u < KQ / 4; u++) {
-        const float4 v = *reinterpret_cast<const float4*>(qs + col * QS + grp * KQ + 4 * u);
+        const float4 v = *reinterpret_cast<const float4*>(qs + col * QS + KU * u + KL * grp);
         qb[4 * u] = v.x; qb[4 * u + 1] = v.y; qb[4 * u + 2] = v.z; qb[4 * u + 3] = v.w;
     }
     const int qpos = (col / G < QT && qt0 + col / G < n_tok) ? pos0 + qt0 + col / G : -1;
@@ -722,28 +776,24 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
     float kr[KQ], vr[4][DT];
     auto load = [&](int kt) {
         const float4* kp = reinterpret_cast<const float4*>(
-            kb + (size_t)min(16 * kt + col, kmax) * kve + grp * KQ);
+            kb + (size_t)min(16 * kt + col, kmax) * kve + KL * grp);
 #pragma unroll
         for (int u = 0; u < KQ / 4; u++) {
-            const float4 v = kp[u];
+            const float4 v = kp[KU / 4 * u];
             kr[4 * u] = v.x; kr[4 * u + 1] = v.y; kr[4 * u + 2] = v.z; kr[4 * u + 3] = v.w;
         }
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const float4* vp = reinterpret_cast<const float4*>(
-                vb + (size_t)min(16 * kt + 4 * grp + r, kmax) * kve + col * DT);
+                vb + (size_t)min(16 * kt + 4 * grp + r, kmax) * kve + 4 * col);
 #pragma unroll
             for (int u = 0; u < DT / 4; u++) {
-                const float4 v = vp[u];
+                const float4 v = vp[16 * u];
                 vr[r][4 * u] = v.x; vr[r][4 * u + 1] = v.y; vr[r][4 * u + 2] = v.z; vr[r][4 * u + 3] = v.w;
             }
         }
     };
-    // head dimension 64: the next tile's rows load during this one; 128: each
-    // tile loads its own (the prefetch registers would leave two waves per SIMD
-    // instead of three: 7B 512-token prefill 22.9 -> 22.7 ms without it, the
-    // Qwen2.5-0.5B shape 5.36 -> 5.41 ms)
-    constexpr bool PF = HD <= 64;
+    // PF: the next tile's rows load during this one
     if (PF && wave < ntile) load(wave);
     for (int kt = wave; kt < ntile; kt += NW) {
         float kc[KQ], vc[4][DT];
@@ -790,12 +840,13 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
     // 2. merge the waves' states (the Q tile is no longer read)
     __syncthreads();
     {
-        float* ow = qs + (wave * R + col) * QS + grp * KQ;  // dims grp*KQ + r*DT + t
+        // tile t, row 4*grp + r: dim 64*(t / 4) + 16*grp + 4*r + t % 4
+        float* ow = qs + (wave * R + col) * QS + 16 * grp;
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
             for (int t4 = 0; t4 < DT / 4; t4++)
-                *reinterpret_cast<float4*>(ow + r * DT + 4 * t4) =
+                *reinterpret_cast<float4*>(ow + 64 * t4 + 4 * r) =
                     make_float4(o[4 * t4][r], o[4 * t4 + 1][r], o[4 * t4 + 2][r], o[4 * t4 + 3][r]);
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
@@ -821,43 +872,16 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
         const float inv = L > 0.f ? 1.f / L : 0.f;
         v = make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);
         // the 8 lanes of a Q8_0 block are consecutive and share r: all store or none
-        if (tl < QT && qt0 + tl < n_tok) {
-            const int t = qt0 + tl;
-            const size_t e0 = (size_t)t * a.out_ld + (size_t)(kvh * G + r % G) * HD + 4 * c4;
-            float* dst = a.out + e0;
-            dst[0] = v.x;
-            dst[1] = v.y;
-            dst[2] = v.z;
-            dst[3] = v.w;
-            if (a.outq8) {
-                const int sub = c4 & 7;
-                float d;
-                const uint32_t p = q8_quant4(v, d);  // q8_store4's block
-                uint8_t* blk = a.outq8 + (e0 >> 5) * Q8_0_BYTES;
-                *reinterpret_cast<uint32_t*>(blk + 4 + 4 * sub) = p;
-                if (sub == 0) *reinterpret_cast<float*>(blk) = d;
-                if (a.xh) {  // k_gemm_prep16's re-layout of the block (out_ld % 32 == 0)
-                    const int kb = (int)((e0 - (size_t)t * a.out_ld) >> 5), Tp = a.Tp;
-                    _Float16 hv[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) hv[e] = (_Float16)(float)(int8_t)(p >> (8 * e));
-                    *reinterpret_cast<uint2*>(a.xh + (((size_t)kb * 4 + (sub >> 1)) * Tp + t) * 16 +
-                                              (sub & 1) * 8) = *reinterpret_cast<const uint2*>(hv);
-                    int sum = dot4((int)p, 0x01010101, 0);
-                    sum += __shfl_xor(sum, 1, 8);
-                    sum += __shfl_xor(sum, 2, 8);
-                    sum += __shfl_xor(sum, 4, 8);
-                    if (sub == 0) {
-                        const size_t i2 = (((size_t)kb * (Tp / 32) + t / 32) * 16 + (t & 15)) * 2 + ((t >> 4) & 1);
-                        const size_t i4 = (((size_t)kb * (Tp / 64) + t / 64) * 16 + (t & 15)) * 4 + ((t >> 4) & 3);
-                        a.dx2[i2] = d;
-                        a.gx2[i2] = d * (float)sum;
-                        a.dx4[i4] = d;
-                    }
-                }
-            }
-        }
+        if (tl < QT && qt0 + tl < n_tok)
+            store_out4<HD>(a, qt0 + tl, kvh * G + r % G, c4, v);
     }
+}
+
+template <int HD, bool PF>
+__global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a, int G, int QT) {
+    __shared__ PrefillKsShared<HD> sh;
+    // longest key ranges first
+    prefill_rows16<HD, PF>(a, G, QT, blockIdx.x, (int)(gridDim.y - 1 - blockIdx.y) * QT, sh);
 }
 
 int attn_nsplit(int max_seq) { return (max_seq + kAttnSplit - 1) / kAttnSplit; }
@@ -868,7 +892,14 @@ static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
     if constexpr (HD <= 128) {
         const int QT = kPfKsRows / G;
         const dim3 grid((unsigned)a.n_kv_heads, (unsigned)((nt + QT - 1) / QT));
-        hipLaunchKernelGGL((k_attn_prefill_ks<HD>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
+        // head dimension 128: prefetch registers leave two waves per SIMD instead of
+        // three, which costs nothing up to one workgroup per CU (32 heads, 33 or 128
+        // tokens on 2000 keys: 84 -> 65 us, 91 -> 73 us with them) and more than the
+        // prefetch brings from two on (16/2 heads, 512 tokens: 120 -> 126 us)
+        if (HD == 64 || grid.x * grid.y <= 256)
+            hipLaunchKernelGGL((k_attn_prefill_ks<HD, true>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
+        else
+            hipLaunchKernelGGL((k_attn_prefill_ks<HD, false>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
         return hipGetLastError();
     }
     const int QT = kPfRows / G;
