@@ -810,6 +810,52 @@ __device__ __forceinline__ void gemm16_step(
     __builtin_amdgcn_s_barrier();
 }
 
+// h of a workgroup's 64 SwiGLU pairs and TW tokens (hs[token][64] in LDS) as
+// Q8_0 blocks of [T][nh] (8 lanes per block, 4 values each, as k_swiglu_gu),
+// fp32 rows with hf, and with hxh k_gemm_prep16's re-layout (zeros past T).
+template <int TW, int THREADS>
+__device__ __forceinline__ void swiglu_blocks(const float* hs, int rt, int tok_base, int nh, int T,
+                                              int Tp, uint8_t* __restrict__ hq8,
+                                              float* __restrict__ hf, uint8_t* __restrict__ hxh,
+                                              float* __restrict__ hdx2, float* __restrict__ hgx2,
+                                              float* __restrict__ hdx4) {
+    for (int q = threadIdx.x; q < TW * 16; q += THREADS) {
+        const int tl = q >> 4, half = (q >> 3) & 1, sub = q & 7, tok = tok_base + tl;
+        if (tok >= Tp) continue;  // the 16 lanes of a token together
+        const float4 o = *reinterpret_cast<const float4*>(hs + tl * 64 + 32 * half + 4 * sub);
+        // the 8 lanes of a block share the token
+        const int kb = 2 * rt + half;  // block of h's row
+        float d = 0.f;
+        uint32_t p = 0u;
+        if (tok < T) {
+            const size_t e = (size_t)tok * nh + 64 * rt + 32 * half + 4 * sub;
+            if (hf) *reinterpret_cast<float4*>(hf + e) = o;
+            p = q8_quant4(o, d);  // q8_block_store's block
+            uint8_t* blk = hq8 + (e >> 5) * Q8_0_BYTES;
+            *reinterpret_cast<uint32_t*>(blk + 4 + 4 * sub) = p;
+            if (sub == 0) *reinterpret_cast<float*>(blk) = d;
+        }
+        if (hxh) {
+            _Float16 hv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) hv[e] = (_Float16)(float)(int8_t)(p >> (8 * e));
+            *reinterpret_cast<uint2*>(hxh + (((size_t)kb * 4 + (sub >> 1)) * Tp + tok) * 16 +
+                                      (sub & 1) * 8) = *reinterpret_cast<const uint2*>(hv);
+            int sum = dot4((int)p, 0x01010101, 0);
+            sum += __shfl_xor(sum, 1, 8);
+            sum += __shfl_xor(sum, 2, 8);
+            sum += __shfl_xor(sum, 4, 8);
+            if (sub == 0) {
+                const size_t i2 = (((size_t)kb * (Tp / 32) + tok / 32) * 16 + (tok & 15)) * 2 + ((tok >> 4) & 1);
+                const size_t i4 = (((size_t)kb * (Tp / 64) + tok / 64) * 16 + (tok & 15)) * 4 + ((tok >> 4) & 3);
+                hdx2[i2] = d;
+                hgx2[i2] = d * (float)sum;
+                hdx4[i4] = d;
+            }
+        }
+    }
+}
+
 // grid = 8 * ceil(nrt / 8) * (Tp / TW) workgroups, XCD-aware: workgroup L runs
 // on XCD L % 8 (round-robin dispatch), and every token group of a row tile
 // runs on one XCD, so the tile's weights are fetched into that XCD's L2 once.
@@ -893,42 +939,7 @@ __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q4k(
             }
         }
         __syncthreads();
-        // 8 lanes per Q8_0 block (4 values each), as k_swiglu_gu: 2 blocks x TW tokens
-        const int nh = rows / 2;
-        for (int q = threadIdx.x; q < TW * 16; q += RT * 64) {
-            const int tl = q >> 4, half = (q >> 3) & 1, sub = q & 7, tok = tok_base + tl;
-            const float4 o = *reinterpret_cast<const float4*>(hs + tl * 64 + 32 * half + 4 * sub);
-            // the 8 lanes of a block share the token
-            const int kb = 2 * rt + half;  // block of h's row
-            float d = 0.f;
-            uint32_t p = 0u;
-            if (tok < T) {
-                const size_t e = (size_t)tok * nh + 64 * rt + 32 * half + 4 * sub;
-                if (hf) *reinterpret_cast<float4*>(hf + e) = o;
-                p = q8_quant4(o, d);  // q8_block_store's block
-                uint8_t* blk = hq8 + (e >> 5) * Q8_0_BYTES;
-                *reinterpret_cast<uint32_t*>(blk + 4 + 4 * sub) = p;
-                if (sub == 0) *reinterpret_cast<float*>(blk) = d;
-            }
-            if (hxh) {  // k_gemm_prep16's re-layout of the block (zeros past T)
-                _Float16 hv[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) hv[e] = (_Float16)(float)(int8_t)(p >> (8 * e));
-                *reinterpret_cast<uint2*>(hxh + (((size_t)kb * 4 + (sub >> 1)) * Tp + tok) * 16 +
-                                          (sub & 1) * 8) = *reinterpret_cast<const uint2*>(hv);
-                int sum = dot4((int)p, 0x01010101, 0);
-                sum += __shfl_xor(sum, 1, 8);
-                sum += __shfl_xor(sum, 2, 8);
-                sum += __shfl_xor(sum, 4, 8);
-                if (sub == 0) {
-                    const size_t i2 = (((size_t)kb * (Tp / 32) + tok / 32) * 16 + (tok & 15)) * 2 + ((tok >> 4) & 1);
-                    const size_t i4 = (((size_t)kb * (Tp / 64) + tok / 64) * 16 + (tok & 15)) * 4 + ((tok >> 4) & 3);
-                    hdx2[i2] = d;
-                    hgx2[i2] = d * (float)sum;
-                    hdx4[i4] = d;
-                }
-            }
-        }
+        swiglu_blocks<TW, RT * 64>(hs, rt, tok_base, rows / 2, T, Tp, hq8, hf, hxh, hdx2, hgx2, hdx4);
         return;
     }
     // a lane's 4 consecutive rows of one token as one 16-byte access where
@@ -943,6 +954,336 @@ __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q4k(
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same product for wide tiles: 4 waves, each 32 weight rows (two row tiles)
+// x 64 tokens (four token tiles), 128 rows x 64 tokens per workgroup.  The
+// kernel is bound by VALU issue: the 16-row waves of k_gemm_f16_q4k rebuild the
+// weight operand for every 32 tokens, 125 of their 212 VALU instructions a
+// block (106 per 16 x 16 tile); here one build serves 64 (82 per tile), and a
+// token fragment read from LDS feeds two MFMAs.  So that two workgroups fit a
+// CU, only the activations (36 KiB a block, two stages) pass through LDS: the
+// weights come as 16-byte loads into registers, one block ahead, turned into
+// the operand layout by the lane-group transpose of k_gemm_q4k_rx.  One barrier
+// a block: a wave's own loads of the block are waited for, then the workgroup
+// meets, then the next block's are issued.  The min term goes into the same
+// accumulator (A = -dmin*m).  Per sub-block the same operations on the same
+// integers as k_gemm_f16_q4k.
+// 512 tokens x 4096, with the activations' quantisation and re-layout:
+// 8192 rows 90.7 -> 74.7 us, 11008 rows 129 -> 111 us, 22016 rows 222 -> 190 us.
+// ---------------------------------------------------------------------------
+struct StageW {
+    static constexpr int RW = 128, TW = 64, NW = 4, NJ = TW / 16;
+    static constexpr int XB = 8 * 4 * TW * 16;  // xh [8 sub-blocks][4][64][16 B]
+    static constexpr int DB = 8 * TW * 4;       // dxt, gxt [8][2][16][2]
+    static constexpr int BYTES = XB + 2 * DB;   // one block: 36 pieces of 1 KiB
+    static_assert(XB == 32 * 1024 && DB == 2048, "pieces 0-31 xh, 32-33 dx, 34-35 gx");
+};
+
+// a row tile's block in registers: header, then bytes 32g..32g+31 of qs
+struct RowBlk {
+    uint4 h, qa, qb;
+};
+
+__device__ __forceinline__ void load_rowblk(RowBlk& b, const uint8_t* p, int g) {
+    b.h = ld16(p);
+    b.qa = ld16(p + 16 + 32 * g);
+    b.qb = ld16(p + 32 + 32 * g);
+}
+
+// the block's operands out of its landing registers
+struct RowOps {
+    uint32_t q[4][2];  // bytes 8g..8g+7 of each 32-byte nibble run
+    uint32_t sc[2];    // the 8 scales
+    float am[2];       // -dmin*m of sub-blocks g and 4 + g
+    float d;
+};
+
+__device__ __forceinline__ void row_ops(RowOps& o, const RowBlk& b, int g) {
+    const uint32_t P[4][2] = {{b.qa.x, b.qa.y}, {b.qa.z, b.qa.w}, {b.qb.x, b.qb.y}, {b.qb.z, b.qb.w}};
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const auto r02 = __builtin_amdgcn_permlane32_swap(P[0][e], P[2][e], false, false);
+        const auto r13 = __builtin_amdgcn_permlane32_swap(P[1][e], P[3][e], false, false);
+        const auto r01 = __builtin_amdgcn_permlane16_swap(r02[0], r13[0], false, false);
+        const auto r23 = __builtin_amdgcn_permlane16_swap(r02[1], r13[1], false, false);
+        o.q[0][e] = r01[0]; o.q[1][e] = r01[1];
+        o.q[2][e] = r23[0]; o.q[3][e] = r23[1];
+    }
+    const uint4 h = b.h;
+    o.sc[0] = h.y & 0x3f3f3f3fu;
+    o.sc[1] = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+    const uint32_t m03 = h.z & 0x3f3f3f3fu;
+    const uint32_t m47 = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+    const float ndmin = -h2f(h.x >> 16);
+    o.am[0] = ndmin * (float)((m03 >> (8 * g)) & 0xffu);
+    o.am[1] = ndmin * (float)((m47 >> (8 * g)) & 0xffu);
+    o.d = h2f(h.x & 0xffffu);
+}
+
+// the A operand of sub-block s: q * sc
+__device__ __forceinline__ v8h_t row_operand(const RowOps& o, int s) {
+    const uint32_t k = (uint32_t)(s & 3);
+    const uint32_t scb = __builtin_amdgcn_perm(0x64646464u, o.sc[s >> 2], 0x04000400u | (k << 16) | k);
+    const h2_t m1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
+    const h2_t sc2 = __builtin_bit_cast(h2_t, scb) + m1024;
+    const h2_t off2 = sc2 * m1024;
+    const int sh = 4 * (s & 1);
+    const uint32_t u0 = (o.q[s >> 1][0] >> sh) & 0x0f0f0f0fu;
+    const uint32_t u1 = (o.q[s >> 1][1] >> sh) & 0x0f0f0f0fu;
+    const u32x4_t aw = {nib_times_sc(u0, 0x04010400u, sc2, off2),
+                        nib_times_sc(u0, 0x04030402u, sc2, off2),
+                        nib_times_sc(u1, 0x04010400u, sc2, off2),
+                        nib_times_sc(u1, 0x04030402u, sc2, off2)};
+    return __builtin_bit_cast(v8h_t, aw);
+}
+
+// A wave's copies of one block: sub-block j's k-group `wave` of the 64 tokens
+// (piece 4j + wave) and a quarter of dx, dx*bsum (piece 32 + wave).  xp, zp:
+// wave-uniform addresses, advanced to the next block; xo, zo: this lane's
+// offsets within a piece.
+__device__ __forceinline__ void copy_block(const uint8_t* __restrict__& xp,
+                                           const uint8_t* __restrict__& zp,
+                                           uint8_t* __restrict__ to, int Tp, int wave, uint32_t xo,
+                                           uint32_t zo) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        __builtin_amdgcn_global_load_lds((gmem_t*)(xp + xo), (lmem_t*)(to + (4 * j + wave) * 1024), 16,
+                                         0, 0);
+        xp += (size_t)Tp * 64;
+    }
+    __builtin_amdgcn_global_load_lds((gmem_t*)(zp + zo), (lmem_t*)(to + (32 + wave) * 1024), 16, 0, 0);
+    zp += (size_t)Tp * 32;
+}
+
+// One block from `cur`, software-pipelined over its sub-blocks: while the matrix
+// core runs sub-block s's 8 products, the VALU applies dx to those of s - 1 and
+// builds the operands of s + 1, about 8 instructions to a product.
+__device__ __forceinline__ void gemmw_block(const uint8_t* __restrict__ cur, const RowOps (&ops)[2],
+                                            int col, int g, v4f_t (&acc)[2][StageW::NJ]) {
+    constexpr int TW = StageW::TW, NJ = StageW::NJ;
+    const uint8_t* xl = cur + (g * TW + col) * 16;
+    const float* dl = reinterpret_cast<const float*>(cur + StageW::XB) + col * 2;
+    const float* gl = dl + 8 * TW;
+    const v4f_t zero = {0.f, 0.f, 0.f, 0.f};
+    v8h_t a[2][2], b[2][NJ];
+    float dx[2][NJ];
+    v4f_t c[2][2][NJ], accb[2][NJ];
+    auto operands = [&](int s) {
+        const int p = s & 1;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            b[p][j] = *reinterpret_cast<const v8h_t*>(xl + (s * 4 * TW + 16 * j) * 16);
+#pragma unroll
+        for (int j = 0; j < NJ; j += 2) {
+            const float2 d = *reinterpret_cast<const float2*>(dl + s * 64 + 16 * j);
+            dx[p][j] = d.x;
+            dx[p][j + 1] = d.y;
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++) a[p][r] = row_operand(ops[r], s);
+    };
+    operands(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s <= 8; s++) {
+        const int p = s & 1, q = p ^ 1;
+        float dq[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) dq[j] = dx[q][j];  // of s - 1, before operands(s + 1) takes them
+        if (s < 8) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    c[p][r][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[p][r], b[p][j], zero, 0, 0, 0);
+        } else {
+            // min term: A = -dmin*m (row col, sub-blocks g and 4 + g), B = d*sum (tokens)
+#pragma unroll
+            for (int j = 0; j < NJ; j += 2) {
+                const float2 g0 = *reinterpret_cast<const float2*>(gl + g * 64 + 16 * j);
+                const float2 g1 = *reinterpret_cast<const float2*>(gl + (4 + g) * 64 + 16 * j);
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ops[r].am[0], g0.x, acc[r][j], 0, 0, 0);
+                    acc[r][j + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ops[r].am[0], g0.y, acc[r][j + 1], 0, 0, 0);
+                    acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ops[r].am[1], g1.x, acc[r][j], 0, 0, 0);
+                    acc[r][j + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ops[r].am[1], g1.y, acc[r][j + 1], 0, 0, 0);
+                }
+            }
+        }
+        if (s < 7) operands(s + 1);
+        if (s > 0) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int ii = 0; ii < 4; ii++)
+                        accb[r][j][ii] = s == 1 ? c[q][r][j][ii] * dq[j]
+                                                : fmaf(c[q][r][j][ii], dq[j], accb[r][j][ii]);
+        }
+        if (s < 8) {
+            __builtin_amdgcn_sched_group_barrier(0x100, NJ + NJ / 2, 0);  // the LDS reads first
+#pragma unroll
+            for (int i = 0; i < 2 * NJ; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            }
+        }
+        // the stage's results belong here: left free, the FMAs drift to the block's
+        // end and hold every product until then
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                if (s < 8) asm volatile("" : "+v"(c[p][r][j]));
+                if (s > 0) asm volatile("" : "+v"(accb[r][j]));
+            }
+            if (s < 7) asm volatile("" : "+v"(a[q][r]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // d of the result rows 4g..4g+3: lane 4g + ii (g = 0 there) holds row 4g + ii's
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        float dout[4];
+#pragma unroll
+        for (int ii = 0; ii < 4; ii++) dout[ii] = __shfl(ops[r].d, 4 * g + ii, 64);
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int ii = 0; ii < 4; ii++) acc[r][j][ii] = fmaf(dout[ii], accb[r][j][ii], acc[r][j][ii]);
+    }
+}
+
+struct WideArgs {
+    float* Y;
+    const uint8_t* W;
+    const uint8_t* xh;
+    const float* dxt;
+    const float* gxt;
+    int rows, nb;
+    long row_bytes;
+    int T, Tp, nrt, accumulate;
+    uint8_t* hq8;  // SwiGLU epilogue (swiglu_blocks)
+    float* hf;
+    uint8_t* hxh;
+    float *hdx2, *hgx2, *hdx4;
+};
+
+// grid as k_gemm_f16_q4k with 64-token groups; Tp % 32 == 0 (a last group of 32
+// repeats its tokens, which are not stored).
+template <bool SW>
+__global__ __launch_bounds__(StageW::NW * 64, 2) void k_gemm_f16_q4k_wide(WideArgs p) {
+    using G = StageW;
+    constexpr int NJ = G::NJ;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * G::BYTES];
+    const int ntg = (p.Tp + G::TW - 1) / G::TW;
+    const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int rt = k / ntg * 8 + xcd, ty = k % ntg;
+    if (rt >= p.nrt) return;  // the whole workgroup, before any barrier
+    const int Tp = p.Tp, nb = p.nb;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, g = lane >> 4;
+    const int row_base = rt * G::RW, tok_base = ty * G::TW;
+    const bool half_group = tok_base + 32 >= Tp;
+    const uint32_t xo = (uint32_t)(half_group ? lane & 31 : lane) * 16;
+    const uint32_t zo = (uint32_t)(lane >> 4) * (uint32_t)(Tp / 32) * 128 +
+                        (half_group ? 0u : (uint32_t)((lane >> 3) & 1) * 128) + (uint32_t)(lane & 7) * 16;
+    const uint8_t* __restrict__ W = p.W;
+    const uint8_t* __restrict__ xp = p.xh + ((size_t)wave * Tp + tok_base) * 16;
+    const uint8_t* __restrict__ zp = reinterpret_cast<const uint8_t*>(wave < 2 ? p.dxt : p.gxt) +
+                                     (size_t)(wave & 1) * Tp * 16 + (size_t)tok_base * 4;
+
+    copy_block(xp, zp, smem, Tp, wave, xo, zo);
+    long wrow[2];  // this lane's rows' blocks, as offsets into W
+    RowBlk blk[2];
+    RowOps ops[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        wrow[r] = (long)min(row_base + 32 * wave + 16 * r + col, p.rows - 1) * p.row_bytes;
+        load_rowblk(blk[r], W + wrow[r], g);
+    }
+    v4f_t acc[2][NJ];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[r][j] = v4f_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < nb; i++) {
+        // every copy of block i is in LDS, and every wave is done with block i - 1
+        wait_vmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int r = 0; r < 2; r++) row_ops(ops[r], blk[r], g);
+        uint8_t* __restrict__ cur = smem + (i & 1) * G::BYTES;
+        uint8_t* __restrict__ nxt = smem + ((i + 1) & 1) * G::BYTES;
+        if (i + 1 < nb) {
+            copy_block(xp, zp, nxt, Tp, wave, xo, zo);
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                wrow[r] += Q4K_BYTES;
+                load_rowblk(blk[r], W + wrow[r], g);
+            }
+        }
+        gemmw_block(cur, ops, col, g, acc);
+    }
+    __syncthreads();  // the ring's LDS is free
+    float* os = reinterpret_cast<float*>(smem);
+    if constexpr (SW) {
+        // lane (col, g < 2) holds gate rows 4g..4g+3 of a row tile's 8 pairs, lane
+        // (col, g + 2) the matching up rows: h[token][64] of this workgroup
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int ii = 0; ii < 4; ii++) {
+                    const float v = acc[r][j][ii], up = __shfl_xor(v, 32, 64);
+                    if (g < 2) os[(16 * j + col) * 64 + 8 * (2 * wave + r) + 4 * g + ii] = swiglu1(v, up);
+                }
+        __syncthreads();
+        swiglu_blocks<G::TW, G::NW * 64>(os, rt, tok_base, p.rows / 2, p.T, Tp, p.hq8, p.hf, p.hxh,
+                                           p.hdx2, p.hgx2, p.hdx4);
+        return;
+    }
+    // through LDS, so that a token's 128 rows leave as 512 contiguous bytes (the
+    // fragments are 64-byte pieces of 16 tokens)
+    constexpr int OS = G::RW + 4;
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            *reinterpret_cast<v4f_t*>(os + (16 * j + col) * OS + 32 * wave + 16 * r + 4 * g) = acc[r][j];
+    __syncthreads();
+    const bool vec = (p.rows & 3) == 0 && ((uintptr_t)p.Y & 15) == 0;
+    for (int i = threadIdx.x; i < G::TW * (G::RW / 4); i += G::NW * 64) {
+        const int t = i / (G::RW / 4), c4 = i % (G::RW / 4), tok = tok_base + t;
+        if (tok < p.T)
+            store_rows4(p.Y + (size_t)tok * p.rows, row_base + 4 * c4, p.rows,
+                        *reinterpret_cast<const v4f_t*>(os + t * OS + 4 * c4), p.accumulate, vec);
+    }
+}
+
+// Where the wide tiles run: from one workgroup per CU on (below, the 32-token
+// groups of k_gemm_f16_q4k leave fewer CUs idle; at exactly 256, 4096 x 4096
+// and 512 tokens, 52.8 -> 51.6 us).
+bool wide_applies(int rows, int T) {
+    return T >= 64 && (long)((rows + 127) / 128) * ((T + 63) / 64) >= 256;
+}
+
+template <bool SW>
+void launch_wide(float* Y, const uint8_t* W, const uint8_t* xh, const float* dxt, const float* gxt,
+                 int rows, int nb, long row_bytes, int T, int Tp, hipStream_t st, int accumulate,
+                 uint8_t* hq8 = nullptr, float* hf = nullptr, uint8_t* hxh = nullptr,
+                 float* hdx2 = nullptr, float* hgx2 = nullptr, float* hdx4 = nullptr) {
+    const int nrt = (rows + StageW::RW - 1) / StageW::RW;
+    const unsigned grid = (unsigned)((nrt + 7) / 8 * 8 * ((Tp + StageW::TW - 1) / StageW::TW));
+    const WideArgs p{Y, W, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, nrt, accumulate,
+                     hq8, hf, hxh, hdx2, hgx2, hdx4};
+    hipLaunchKernelGGL(k_gemm_f16_q4k_wide<SW>, dim3(grid), dim3(StageW::NW * 64), 0, st, p);
+}
+
 template <int RT, int TTW, int S>
 void launch16_cfg(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scratch, int rows,
                   int nb, long row_bytes, int T, hipStream_t st, int accumulate) {
@@ -954,6 +1295,10 @@ void launch16_cfg(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scrat
     const long n = (long)nkb * Tp;
     hipLaunchKernelGGL(k_gemm_prep16<TTW>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                        XQ8, T, Tp, nkb, xh, dxt, gxt);
+    if (wide_applies(rows, T)) {
+        launch_wide<false>(Y, W, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, accumulate);
+        return;
+    }
     const int nrt = (rows + kTile * RT - 1) / (kTile * RT);
     const unsigned grid = (unsigned)((nrt + 7) / 8 * 8 * (Tp / TW));
     hipLaunchKernelGGL((k_gemm_f16_q4k<RT, TTW, S>), dim3(grid), dim3(RT * 64), 0, st, Y, W, xh,
@@ -1603,9 +1948,17 @@ hipError_t launch_gemm_f16_q4k_xh(float* Y, uint8_t* hq8, float* hf, const void*
     if (rows <= 0 || nb <= 0 || T <= 0 || Tp < T || Tp % TW || (swiglu && rows % 128) ||
         (hxh && (Tp % 64 || !hdx2 || !hgx2 || !hdx4)))
         return hipErrorInvalidValue;
+    const auto* w = static_cast<const uint8_t*>(W);
+    if (wide_applies(rows, T)) {
+        if (swiglu)
+            launch_wide<true>(nullptr, w, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, 0, hq8, hf,
+                              hxh, hdx2, hgx2, hdx4);
+        else
+            launch_wide<false>(Y, w, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, accumulate);
+        return hipGetLastError();
+    }
     const int nrt = (rows + kTile * RT - 1) / (kTile * RT);
     const unsigned grid = (unsigned)((nrt + 7) / 8 * 8 * (Tp / TW));
-    const auto* w = static_cast<const uint8_t*>(W);
     if (swiglu)
         hipLaunchKernelGGL((k_gemm_f16_q4k<RT, TTW, S, true>), dim3(grid), dim3(RT * 64), 0, st,
                            nullptr, w, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, nrt, 0, hq8, hf,

@@ -1,0 +1,34 @@
+"""The wide-tile Q4_K GEMM (128 rows x 64 tokens per workgroup) at its edges:
+a last token group of 32, ragged rows and tokens, one super-block of K, and the
+smallest grid it takes, against the oracle's per-token GEMV."""
+import numpy as np
+import pytest
+
+from llm_core_amd import hip
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,T", [
+    (32768, 256, 65),     # 256 x 2 groups, the second of one token (Tp % 64 == 32), one super-block
+    (16385, 512, 97),     # a last row tile of one row, 33 tokens in the last group
+    (8191, 1024, 256),    # rows % 4 != 0: per-row stores
+    (4096, 512, 512),     # exactly 256 workgroups
+    (4224, 768, 491),     # 33 row tiles: XCD 0 has one more than the others
+])
+def test_gemm_wide(ctx, rows, cols, T):
+    W = hip.synth_weight(12, rows, cols, seed=rows + T)
+    X = hip.synth_normal(T * cols, seed=7)
+    xq = O.quantize_q8_0(X)
+    y = ctx.alloc(T * rows * 4)
+    ctx.write(y, np.full(T * rows, np.nan, np.float32))
+    ctx.gemm_q4k_q8(y, ctx.upload(W), ctx.upload(xq), rows, T, cols, hip.row_bytes(12, cols))
+    got = ctx.download(y, np.float32, T * rows).reshape(T, rows)
+    assert np.isfinite(got).all()
+    nb = cols // 32 * 36
+    for t in sorted({0, 1, 31, 32, 63, 64, T // 2, T - 1}):
+        want = O.gemv_q8(12, W, xq[t * nb:(t + 1) * nb], rows, cols).astype(np.float64)
+        # fp32 sums of cols / 32 + cols / 256 terms in another order
+        tol = (cols // 32 + cols // 256 + 8) * 2.0 ** -24 * np.abs(want).max() * 8
+        assert np.max(np.abs(got[t] - want)) <= tol, (t, np.max(np.abs(got[t] - want)), tol)
