@@ -116,7 +116,9 @@ hipError_t launch_gemm_stream_q4k_q8(float* Y, const void* W, const void* XQ8, i
 hipError_t launch_gemm_mfma_q4k_q8(float* Y, const void* W, const void* XQ8, int rows, int T,
                                    int nb, long row_bytes, void* scratch, hipStream_t st,
                                    int accumulate = 0);
-size_t gemm_mfma_q6k_scratch_bytes(int T, int nb);
+size_t gemm_mfma_q6k_scratch_bytes(int T, int nb, int rows);
+// the most that any matrix needs for up to T tokens
+size_t gemm_mfma_q6k_max_scratch_bytes(int T, int nb);
 // The fp16 GEMMs on a re-layout written elsewhere (launch_rmsnorm_rows_prep):
 // xh / dxt / gxt as k_gemm_prep16 lays them out for Tp tokens (a multiple of
 // 64 serves both).  Q6_K: where gemm_f16_q6k_applies.  Q4_K with swiglu: the

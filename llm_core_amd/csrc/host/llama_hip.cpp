@@ -710,6 +710,10 @@ int prefill_alloc(axf_llama* m) {
                 const size_t b = gemm_scratch_bytes(qt, GemmPath::Auto, t, kmax / QK_K, rmax);
                 if (b > gs) gs = b;
             }
+    {  // the Q6_K GEMM's K ranges: more of them for fewer tokens
+        const size_t qs = gemm_mfma_q6k_max_scratch_bytes(cap, (kmax > qo ? kmax : qo) / QK_K);
+        if (gs < qs) gs = qs;
+    }
     {  // the misc GEMM's hi/lo rows
         const size_t ms = gemm_misc_scratch_bytes(cap, kmax > qo ? kmax : qo);
         if (gs < ms) gs = ms;

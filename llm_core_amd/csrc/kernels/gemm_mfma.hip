@@ -1640,7 +1640,7 @@ __device__ __forceinline__ void bytes_scaled(uint32_t u, h2_t off2, h2_t sc2, ui
 template <int RT, int TTW, int S>
 __device__ __forceinline__ void gemm6h_step(
     const uint8_t* __restrict__ cur, uint8_t* __restrict__ nxt, bool do_copy, int bnext, int i,
-    int nb, const uint64_t (&base)[Stage6h<RT, TTW, S>::PMAX],
+    int nb, int b0, const uint64_t (&base)[Stage6h<RT, TTW, S>::PMAX],
     const uint32_t (&aux)[Stage6h<RT, TTW, S>::PMAX], __amdgpu_buffer_rsrc_t wrsrc, int wave,
     int col, int g, uint32_t wlo, v4f_t (&acc)[TTW]) {
     using G = Stage6h<RT, TTW, S>;
@@ -1666,9 +1666,9 @@ __device__ __forceinline__ void gemm6h_step(
     wait_later<G::PMIN, S - 1>(min(S - 1, nb - 1 - i));
     __builtin_amdgcn_s_barrier();
 
-    // this lane's row: its block starts (wlo + 2i) & 15 bytes into the slot
+    // this lane's row: its block b0 + i starts (wlo + 2 (b0 + i)) & 15 bytes into the slot
     const uint8_t* wl = cur + (kTile * wave + col) * G::SLOT;
-    const uint32_t wo = (wlo + 2u * (uint32_t)i) & 15u;
+    const uint32_t wo = (wlo + 2u * (uint32_t)(b0 + i)) & 15u;
     const uint8_t* xl = cur + G::WB;
     const float* dl = reinterpret_cast<const float*>(cur + G::WB + G::XB);
     uint32_t ql[2][2][2], qh[2][2], sc[4], dw[1];
@@ -1728,12 +1728,14 @@ __device__ __forceinline__ void gemm6h_step(
     __builtin_amdgcn_s_barrier();
 }
 
-// grid = 8 * ceil(nrt / 8) * (Tp / TW) workgroups, XCD-aware as k_gemm_f16_q4k
+// grid.x = 8 * ceil(nrt / 8) * (Tp / TW) workgroups, XCD-aware as k_gemm_f16_q4k.
+// grid.y ranges of kper super-blocks: with more than one, range y's sums go to
+// part[y][T][rows] (k_gemm_splitk_add adds them in order) instead of Y.
 template <int RT, int TTW, int S>
 __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q6k(
-    float* __restrict__ Y, const uint8_t* __restrict__ W, const uint8_t* __restrict__ xh,
+    float* Y, const uint8_t* __restrict__ W, const uint8_t* __restrict__ xh,
     const float* __restrict__ dxt, int rows, int nb, long row_bytes, int T, int Tp, int nrt,
-    int accumulate) {
+    int accumulate, int kper, float* __restrict__ part) {
     using G = Stage6h<RT, TTW, S>;
     constexpr int NW = G::NW, RW = G::RW, TW = G::TW;
     __shared__ __attribute__((aligned(16))) uint8_t smem[S * G::ALLOC];
@@ -1784,11 +1786,16 @@ __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q6k(
     v4f_t acc[TTW];
 #pragma unroll
     for (int j = 0; j < TTW; j++) acc[j] = v4f_t{0.f, 0.f, 0.f, 0.f};
-    for (int i = 1 - S; i < nb; i++) {
+    const int b0 = (int)blockIdx.y * kper, n = min(kper, nb - b0);
+    for (int i = 1 - S; i < n; i++) {
         const int inext = i + S - 1;
         gemm6h_step<RT, TTW, S>(smem + ((i + S) % S) * G::ALLOC, smem + (inext % S) * G::ALLOC,
-                                inext < nb, inext, i, nb, base, aux, wrsrc, wave, col, g, wlo,
+                                inext < n, b0 + inext, i, n, b0, base, aux, wrsrc, wave, col, g, wlo,
                                 acc);
+    }
+    if (gridDim.y > 1) {
+        Y = part + (size_t)blockIdx.y * T * rows;
+        accumulate = 0;
     }
     const bool vec = (rows & 3) == 0 && ((uintptr_t)Y & 15) == 0;
 #pragma unroll
@@ -1803,6 +1810,55 @@ __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q6k(
 // two 64 KiB stages)
 constexpr int kF16Q6RT = 8, kF16Q6TTW = 4, kF16Q6S = 2;
 
+// K ranges of the fp16 kernel (a CU holds one workgroup): one from 192 tiles of
+// 128 x 64 up, below that as many as fit 256 workgroups; 0: the int8 kernel's
+// small tiles instead.  Those scale every result on the VALU, but fill the chip
+// by themselves and store no partial sums: ranges pay from 3 super-blocks on,
+// and where 64 x 64 tiles fill the chip already (128 tiles of ours) from 12.
+// With the activations' quantisation and re-layout, int8 -> here: 4096 x 11008
+// at 64 tokens 41.9 -> 38.4 us, at 100 75.9 -> 56.1, 2048 x 11008 at 200
+// 76.1 -> 56.5, 4096 x 11008 at 400 (224 tiles, one range) 197 -> 166.  Below
+// the lines: 4096 x 4096 at 64 tokens (2 super-blocks a range) 18.9 -> 23.0,
+// 4096 x 2048 at 200 (128 tiles, 4) 25.3 -> 29.3.
+int q6_ranges(int rows, int T, int nb, int* kper) {
+    *kper = nb;
+    if (T <= 32) return 0;  // 64-token tiles would be half empty
+    const long tiles = (long)((rows + 127) / 128) * ((T + 63) / 64);
+    if (tiles >= 192) return 1;
+    const int want = (int)(256 / tiles);
+    if (want == 1) return 0;
+    *kper = (nb + want - 1) / want;
+    return *kper >= (tiles >= 128 ? 12 : 3) ? (nb + *kper - 1) / *kper : 0;
+}
+
+// partial sums: at most 256 tiles of 128 x 64
+constexpr size_t kF16Q6SplitBytes = (size_t)256 * 128 * 64 * sizeof(float);
+
+size_t q6_split_bytes(int rows, int T, int nb) {
+    int kper;
+    const int n = q6_ranges(rows, T, nb, &kper);
+    return n > 1 ? (size_t)n * T * rows * sizeof(float) : 0;
+}
+
+// Y[i] (+)= part[0][i] + part[1][i] + ... (n values each, n % 4 == 0 when vec)
+__global__ __launch_bounds__(256) void k_gemm_splitk_add(float* __restrict__ Y,
+                                                         const float* __restrict__ part, size_t n,
+                                                         int ranges, int accumulate, int vec) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * (vec ? 4 : 1);
+    if (i >= n) return;
+    if (!vec) {
+        float s = part[i];
+        for (int k = 1; k < ranges; k++) s += part[k * n + i];
+        Y[i] = accumulate ? Y[i] + s : s;
+        return;
+    }
+    v4f_t s = *reinterpret_cast<const v4f_t*>(part + i);
+#pragma unroll 4
+    for (int k = 1; k < ranges; k++) s += *reinterpret_cast<const v4f_t*>(part + k * n + i);
+    v4f_t* y = reinterpret_cast<v4f_t*>(Y + i);
+    *y = accumulate ? *y + s : s;
+}
+
 void launch6h(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scratch, int rows, int nb,
               long row_bytes, int T, hipStream_t st, int accumulate) {
     constexpr int TW = kTile * kF16Q6TTW;
@@ -1810,14 +1866,24 @@ void launch6h(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scratch, 
     auto* xh = scratch;
     auto* dxt = reinterpret_cast<float*>(xh + (size_t)nkb * Tp * 64);
     auto* gxt = dxt + (size_t)nkb * Tp;  // written by the shared re-layout, unused here
+    float* part = gxt + (size_t)nkb * Tp;
     const long n = (long)nkb * Tp;
     hipLaunchKernelGGL(k_gemm_prep16<kF16Q6TTW>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        st, XQ8, T, Tp, nkb, xh, dxt, gxt);
     const int nrt = (rows + kTile * kF16Q6RT - 1) / (kTile * kF16Q6RT);
     const unsigned grid = (unsigned)((nrt + 7) / 8 * 8 * (Tp / TW));
-    hipLaunchKernelGGL((k_gemm_f16_q6k<kF16Q6RT, kF16Q6TTW, kF16Q6S>), dim3(grid),
+    int kper;
+    const int ranges = q6_ranges(rows, T, nb, &kper);
+    hipLaunchKernelGGL((k_gemm_f16_q6k<kF16Q6RT, kF16Q6TTW, kF16Q6S>), dim3(grid, (unsigned)ranges),
                        dim3(kF16Q6RT * 64), 0, st, Y, W, xh, dxt, rows, nb, row_bytes, T, Tp, nrt,
-                       accumulate);
+                       accumulate, kper, part);
+    if (ranges > 1) {
+        const size_t m = (size_t)T * rows;
+        const int vec = m % 4 == 0 && (((uintptr_t)Y | (uintptr_t)part) & 15) == 0;
+        const size_t per = vec ? 1024 : 256;
+        hipLaunchKernelGGL(k_gemm_splitk_add, dim3((unsigned)((m + per - 1) / per)), dim3(256), 0, st,
+                           Y, part, m, ranges, accumulate, vec);
+    }
 }
 
 // Tile choice: the largest of 64x64, 32x32, 16x16 (rows x tokens) whose grid
@@ -1882,10 +1948,16 @@ bool gemm_mfma_q6k_ok(const void* W, int rows, int nb, long row_bytes) {
     return bytes + 16 < (1ull << 31) && ((reinterpret_cast<uintptr_t>(W) + bytes) & 15) == 0;
 }
 
-size_t gemm_mfma_q6k_scratch_bytes(int T, int nb) {
-    if (T <= 0 || nb <= 0) return 0;
+size_t gemm_mfma_q6k_scratch_bytes(int T, int nb, int rows) {
+    if (T <= 0 || nb <= 0 || rows <= 0) return 0;
     const size_t tp = (size_t)((T + 63) / 64 * 64);  // the widest token tile's padding
-    return (size_t)nb * 8 * tp * (64 + 4 + 4);        // fp16 re-layout (int8: 32 + 4 + 4)
+    // fp16 re-layout (int8: 32 + 4 + 4), then the K ranges' partial sums
+    return (size_t)nb * 8 * tp * (64 + 4 + 4) + q6_split_bytes(rows, T, nb);
+}
+
+size_t gemm_mfma_q6k_max_scratch_bytes(int T, int nb) {
+    if (T <= 0 || nb <= 0) return 0;
+    return (size_t)nb * 8 * ((T + 63) / 64 * 64) * (64 + 4 + 4) + kF16Q6SplitBytes;
 }
 
 hipError_t launch_gemm_mfma_q6k_q8(float* Y, const void* W, const void* XQ8, int rows, int T,
@@ -1893,9 +1965,7 @@ hipError_t launch_gemm_mfma_q6k_q8(float* Y, const void* W, const void* XQ8, int
                                    int accumulate) {
     if (rows <= 0 || T <= 0 || nb <= 0 || scratch == nullptr) return hipErrorInvalidValue;
     if (!gemm_mfma_q6k_ok(W, rows, nb, row_bytes)) return hipErrorInvalidValue;
-    // wide token tiles on the fp16 matrix cores where 128 x 64 tiles still give
-    // one workgroup per CU
-    if (gemm_f16_q6k_applies(W, rows, nb, row_bytes, T)) {
+    if (int kper; q6_ranges(rows, T, nb, &kper)) {
         launch6h(Y, static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(XQ8),
                  static_cast<uint8_t*>(scratch), rows, nb, row_bytes, T, st, accumulate);
         return hipGetLastError();
@@ -1984,7 +2054,7 @@ hipError_t launch_gemm_f16_q6k_xh(float* Y, const void* W, const uint8_t* xh, co
     const unsigned grid = (unsigned)((nrt + 7) / 8 * 8 * (Tp / TW));
     hipLaunchKernelGGL((k_gemm_f16_q6k<kF16Q6RT, kF16Q6TTW, kF16Q6S>), dim3(grid),
                        dim3(kF16Q6RT * 64), 0, st, Y, static_cast<const uint8_t*>(W), xh, dxt,
-                       rows, nb, row_bytes, T, Tp, nrt, accumulate);
+                       rows, nb, row_bytes, T, Tp, nrt, accumulate, nb, (float*)nullptr);
     return hipGetLastError();
 }
 

@@ -1612,7 +1612,7 @@ GemmPath gemm_resolve(GemmPath path, int T) {
 size_t gemm_scratch_bytes(int qtype, GemmPath path, int T, int nb, int rows) {
     const GemmPath p = gemm_resolve(path, T);
     if (p == GemmPath::Dot4) return 0;
-    if (qtype == AXF_TYPE_Q6_K) return gemm_mfma_q6k_scratch_bytes(T, nb);
+    if (qtype == AXF_TYPE_Q6_K) return gemm_mfma_q6k_scratch_bytes(T, nb, rows);
     const size_t mf = gemm_mfma_scratch_bytes(T, nb);
     if (p == GemmPath::Stream && gemm_stream_q4k_ok(T, nb, rows)) {
         // room for the Mfma fallback (unaligned operands) as well

@@ -27,8 +27,34 @@ def test_gemm_wide(ctx, rows, cols, T):
     got = ctx.download(y, np.float32, T * rows).reshape(T, rows)
     assert np.isfinite(got).all()
     nb = cols // 32 * 36
-    for t in sorted({0, 1, 31, 32, 63, 64, T // 2, T - 1}):
+    for t in sorted({t for t in (0, 1, 31, 32, 63, 64, T // 2, T - 1) if t < T}):
         want = O.gemv_q8(12, W, xq[t * nb:(t + 1) * nb], rows, cols).astype(np.float64)
+        # fp32 sums of cols / 32 + cols / 256 terms in another order
+        tol = (cols // 32 + cols // 256 + 8) * 2.0 ** -24 * np.abs(want).max() * 8
+        assert np.max(np.abs(got[t] - want)) <= tol, (t, np.max(np.abs(got[t] - want)), tol)
+
+
+@pytest.mark.parametrize("rows,cols,T", [
+    (4096, 6144, 33),     # 8 ranges of 3 super-blocks, the shortest taken
+    (1000, 10240, 70),    # ragged rows and tokens, 14 ranges, the last of one super-block
+    (1024, 11008, 65),    # 8 row tiles x 2 groups, 43 super-blocks in 15 ranges
+    (2048, 6144, 512),    # 128 tiles: 2 ranges of 12
+    (24640, 512, 40),     # 193 tiles, one range
+])
+def test_gemm_q6k_ranges(ctx, rows, cols, T):
+    W = hip.synth_weight(14, rows, cols, seed=rows + T)
+    if (rows * hip.row_bytes(14, cols)) % 16:
+        pytest.skip("the last block does not end on a 16-byte boundary: the dot4 kernel")
+    X = hip.synth_normal(T * cols, seed=9)
+    xq = O.quantize_q8_0(X)
+    y = ctx.alloc(T * rows * 4)
+    ctx.write(y, np.full(T * rows, np.nan, np.float32))
+    ctx.gemm_q6k_q8(y, ctx.upload(W), ctx.upload(xq), rows, T, cols, hip.row_bytes(14, cols))
+    got = ctx.download(y, np.float32, T * rows).reshape(T, rows)
+    assert np.isfinite(got).all()
+    nb = cols // 32 * 36
+    for t in sorted({t for t in (0, 31, 32, 63, T // 2, T - 1) if t < T}):
+        want = O.gemv_q8(14, W, xq[t * nb:(t + 1) * nb], rows, cols).astype(np.float64)
         # fp32 sums of cols / 32 + cols / 256 terms in another order
         tol = (cols // 32 + cols // 256 + 8) * 2.0 ** -24 * np.abs(want).max() * 8
         assert np.max(np.abs(got[t] - want)) <= tol, (t, np.max(np.abs(got[t] - want)), tol)
