@@ -884,12 +884,433 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
     prefill_rows16<HD, PF>(a, G, QT, blockIdx.x, (int)(gridDim.y - 1 - blockIdx.y) * QT, sh);
 }
 
+// ---------------------------------------------------------------------------
+// The same attention on the fp16 matrix cores, fp32 kept by splitting: a tile's
+// values are scaled by a power of two so that the largest is in [2^14, 2^15)
+// and written as x = h + l, two fp16 parts rounded one after the other (22 bits
+// and the sign of l: 2^-23 of x, for values down to 2^-15 of the largest;
+// 2^-40 of the largest below).  A product is hh + hl + lh, accumulated in fp32,
+// the small ones first; ll is under 2^-24 of it.  v_mfma_f32_16x16x32_f16 does
+// 8x the products of v_mfma_f32_16x16x4_f32 in half its cycles, so three of
+// them cost 3/16.
+//
+// A workgroup owns 64 query rows of one kv head (QT = 64 / G tokens x the G
+// heads that share it): 4 key groups x 2 waves of 32 rows, two waves per SIMD.
+// Group kg takes the 32-key tiles kt = kg, kg + 4, ...; its two waves load the
+// tile's K and V rows (the next tile's while this one is computed), split them
+// once for all 64 rows and put the parts into LDS in operand order, where they
+// are read as conflict-free 16-byte fragments.  Q's parts stay in registers.
+// Splitting and the softmax are the VALU work beside the products; the 16-row
+// workgroups of k_attn_prefill_ks would split every K/V element four times as
+// often, and a splitting pass of its own would move 2x the K/V bytes first.
+//   S^T = K Q^T  A = 16 keys x 32 dims, B = 16 query rows; result lane (col,
+//                g): keys 4g + r of query col.
+//   O^T = V^T P^T  A = 16 dims x 32 keys, B = P as the two S^T tiles hold it:
+//                k-slot e of lane group g is key 4g + e (e < 4) or 16 + 4g +
+//                e - 4; tile t's row c is dim DT*c + t, so a result lane
+//                holds DT consecutive dims.
+// The running maximum is kept as a whole power of two, M = ceil(max * log2(e)
+// / sqrt(HD)): p = 2^(s * c - M) is one fma and one v_exp_f32, and rescaling by
+// 2^(M_old - M_new) is exact, as are the tiles' scales.
+// 32 heads of 128, 512 tokens at position 1536: error against 64 bits 5.6e-7
+// with fp32 products, 3.4e-7 here; 183 -> 143 us (15 GFLOP, 105 TFLOP/s).
+//
+// The scales cover tiles whose largest |x| is in [2^-40, 2^40) or 0.  A
+// workgroup that meets another (infinities, say) computes its rows again with
+// k_attn_prefill_ks's arithmetic.
+// ---------------------------------------------------------------------------
+constexpr int kPfSpRows = 64;    // query rows per workgroup
+constexpr int kPfSpKeys = 32;    // keys per tile
+constexpr int kPfSpGroups = 4;   // key groups
+constexpr int kPfSpThreads = kPfSpGroups * 128;
+
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
+
+// x * s for 8 floats as two 8-element operands h + l
+__device__ __forceinline__ void split2x8(const float (&x)[8], float s, uint4& h, uint4& l) {
+    uint32_t ph[4], pl[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = x[2 * i], b = x[2 * i + 1];
+        const h2_t hh = {(_Float16)(a * s), (_Float16)(b * s)};
+        const h2_t lo = {(_Float16)fmaf(a, s, -(float)hh.x), (_Float16)fmaf(b, s, -(float)hh.y)};
+        ph[i] = __builtin_bit_cast(uint32_t, hh);
+        pl[i] = __builtin_bit_cast(uint32_t, lo);
+    }
+    h = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+    l = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+}
+
+__device__ __forceinline__ bool split_range(float amax) {
+    return amax == 0.f || (amax >= 0x1p-40f && amax < 0x1p40f);
+}
+
+// e with amax * 2^e in [2^14, 2^15) (0 for amax = 0), for amax in split_range
+__device__ __forceinline__ int split_exp(float amax) {
+    return amax == 0.f ? 0 : 14 + 127 - (int)(__float_as_uint(amax) >> 23);
+}
+__device__ __forceinline__ float pow2i(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
+
+__device__ __forceinline__ v4f_t mfma_h(const uint4& a, const uint4& b, v4f_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h_t, a),
+                                                  __builtin_bit_cast(v8h_t, b), c, 0, 0, 0);
+}
+
+// max of v over the lanes l ^ 16, l ^ 32 and l ^ 48
+__device__ __forceinline__ float max_over_groups(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+template <int HD>
+struct PrefillSpShared {
+    static constexpr int KS = HD / 32, DT = HD / 16;
+    static constexpr int QS = HD + 4;
+    union {
+        // per key group: K [key tile 2][k-step][part] and V [dim tile][part],
+        // 64 x 16 bytes each
+        struct {
+            uint4 k[kPfSpGroups][2 * KS * 2 * 64];
+            uint4 v[kPfSpGroups][DT * 2 * 64];
+        };
+        float o[kPfSpGroups * kPfSpRows * QS];  // the Q rows, then the groups' O rows
+        PrefillKsShared<HD> ks;
+    };
+    float am[kPfSpGroups][2][2];  // the next tile's largest |K| and |V| per wave
+    float mm[kPfSpGroups][kPfSpRows], ll[kPfSpGroups][kPfSpRows];
+    int ve[kPfSpGroups][2];       // each wave's last V exponent
+    int redo;
+};
+
+template <int HD>
+__global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, int G, int QT) {
+    using SH = PrefillSpShared<HD>;
+    constexpr int KS = SH::KS, DT = SH::DT, QS = SH::QS, HALF = HD / 2;
+    constexpr int R = kPfSpRows, NG = kPfSpGroups, VD = HD / 32;  // VD: dims of V per loading lane
+    __shared__ SH sh;
+
+    const int kvh = blockIdx.x;
+    const int qt0 = (int)(gridDim.y - 1 - blockIdx.y) * QT;  // longest key ranges first
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, grp = lane >> 4;
+    // key group, 32-row block: a SIMD's two waves share their tiles
+    const int kg = wave & (kPfSpGroups - 1), qb = wave / kPfSpGroups;
+    const int pos0 = a.pos_dev ? *a.pos_dev : a.pos;
+    const int n_tok = a.n_tok > 1 ? a.n_tok : 1;
+    const int t_end = min(qt0 + QT, n_tok);
+    const int kmax = pos0 + t_end - 1;  // last key any row attends to
+    const size_t kve = (size_t)a.n_kv_heads * HD;
+    const float* kb = a.kcache + (size_t)kvh * HD;
+    const float* vb = a.vcache + (size_t)kvh * HD;
+    const int ntile = kmax / kPfSpKeys + 1;
+
+    // the tile's K and V rows as this thread splits them: K key 16*qb + col,
+    // dims 32*s + 4*grp .. +3 and 16 above those (one load covers 64 contiguous
+    // bytes of a row); V keys of k-slots 0..7 of group vg, dims VD*dg ..  Rows
+    // are byte offsets, clamped to row kmax (keys past it are masked below).
+    const int vi = qb * 64 + lane, vg = vi >> 5, dg = 2 * (vi & 15) + ((vi >> 4) & 1);
+    const uint32_t rowb = (uint32_t)kve * 4, lim = (uint32_t)kmax * rowb;
+    uint32_t ko = (uint32_t)(kPfSpKeys * kg + 16 * qb + col) * rowb;
+    uint32_t vo = (uint32_t)(kPfSpKeys * kg + 4 * vg) * rowb;
+    const char* kp = reinterpret_cast<const char*>(kb + 4 * grp);
+    const char* vp = reinterpret_cast<const char*>(vb + VD * dg);
+    float kr[KS][8], vr[8][VD];
+    auto load = [&] {  // the group's next tile
+        const char* k = kp + min(ko, lim);
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const float4 x = *reinterpret_cast<const float4*>(k + 128 * s);
+            const float4 y = *reinterpret_cast<const float4*>(k + 128 * s + 64);
+            kr[s][0] = x.x; kr[s][1] = x.y; kr[s][2] = x.z; kr[s][3] = x.w;
+            kr[s][4] = y.x; kr[s][5] = y.y; kr[s][6] = y.z; kr[s][7] = y.w;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const char* v = vp + min(vo + (uint32_t)(e < 4 ? e : 12 + e) * rowb, lim);
+            if constexpr (VD == 4) {
+                const float4 x = *reinterpret_cast<const float4*>(v);
+                vr[e][0] = x.x; vr[e][1] = x.y; vr[e][2] = x.z; vr[e][3] = x.w;
+            } else {
+                const float2 x = *reinterpret_cast<const float2*>(v);
+                vr[e][0] = x.x; vr[e][1] = x.y;
+            }
+        }
+        ko += (uint32_t)(kPfSpKeys * NG) * rowb;
+        vo += (uint32_t)(kPfSpKeys * NG) * rowb;
+    };
+    // the loaded rows' largest magnitudes, for both waves to agree on the scale
+    auto publish_max = [&] {
+        float mk = 0.f, mv = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) mk = fmaxf(mk, fabsf(kr[s][e]));
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+#pragma unroll
+            for (int j = 0; j < VD; j++) mv = fmaxf(mv, fabsf(vr[e][j]));
+        mk = wave_max_bcast(mk);
+        mv = wave_max_bcast(mv);
+        if (lane == 0) {
+            sh.am[kg][qb][0] = mk;
+            sh.am[kg][qb][1] = mv;
+        }
+    };
+    if (kg < ntile) load();
+
+    // 1. Q rows: row r = token qt0 + r / G, head kvh*G + r % G (+ bias, RoPE)
+    for (int idx = tid; idx < R * HD; idx += kPfSpThreads) {
+        const int r = idx / HD, d = idx % HD, tl = r / G;
+        float v = 0.f;
+        if (tl < QT && qt0 + tl < n_tok) {
+            const size_t e = (size_t)(kvh * G + r % G) * HD + d;
+            v = a.q[(size_t)(qt0 + tl) * a.q_ld + e];
+            if (a.bq) v += a.bq[e];
+        }
+        sh.o[r * QS + d] = v;
+    }
+    if (tid == 0) sh.redo = 0;
+    __syncthreads();
+    if (a.cos_t) {
+        for (int idx = tid; idx < R * HALF; idx += kPfSpThreads) {
+            const int r = idx / HALF, i = idx % HALF, tl = r / G;
+            if (tl < QT && qt0 + tl < n_tok) {
+                const size_t pr = (size_t)(pos0 + qt0 + tl) * HALF + i;
+                const float c = a.cos_t[pr], sn = a.sin_t[pr];
+                float* h = sh.o + r * QS;
+                const float x0 = h[i], x1 = h[i + HALF];
+                h[i] = fmaf(x0, c, -(x1 * sn));
+                h[i + HALF] = fmaf(x0, sn, x1 * c);
+            }
+        }
+        __syncthreads();
+    }
+    // B of S^T: query row 32*qb + 16*j + col, the dims of K's operands
+    uint4 qp[2][KS][2];
+    bool fine;
+    float c;  // log2(e) / sqrt(HD) over the Q scale
+    {
+        float qv[2][KS][8], mq = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const float* p = sh.o + (32 * qb + 16 * j + col) * QS + 32 * s + 4 * grp;
+                const float4 x = *reinterpret_cast<const float4*>(p);
+                const float4 y = *reinterpret_cast<const float4*>(p + 16);
+                qv[j][s][0] = x.x; qv[j][s][1] = x.y; qv[j][s][2] = x.z; qv[j][s][3] = x.w;
+                qv[j][s][4] = y.x; qv[j][s][5] = y.y; qv[j][s][6] = y.z; qv[j][s][7] = y.w;
+#pragma unroll
+                for (int e = 0; e < 8; e++) mq = fmaxf(mq, fabsf(qv[j][s][e]));
+            }
+        mq = wave_max_bcast(mq);
+        fine = split_range(mq);
+        const int e = fine ? split_exp(mq) : 0;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int s = 0; s < KS; s++) split2x8(qv[j][s], pow2i(e), qp[j][s][0], qp[j][s][1]);
+        c = 1.44269504088896341f / sqrtf((float)HD) * pow2i(-e);
+    }
+    int qpos[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int tl = (32 * qb + 16 * j + col) / G;
+        qpos[j] = (tl < QT && qt0 + tl < n_tok) ? pos0 + qt0 + tl : -1;
+    }
+    // this wave's first and last token (rows 32*qb ..)
+    const int wave_lo = pos0 + qt0 + 32 * qb / G;
+    const int wave_hi = min(pos0 + qt0 + (32 * qb + 31) / G, kmax);
+    const bool wave_rows = 32 * qb / G < QT && qt0 + 32 * qb / G < n_tok;
+
+    float M[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+    int ve = 0;  // o is in units of 2^-ve
+    v4f_t o[2][DT];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int t = 0; t < DT; t++) o[j][t] = v4f_t{0.f, 0.f, 0.f, 0.f};
+
+    const v4f_t zero = {0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < (ntile + NG - 1) / NG; it++) {
+        const int kt = NG * it + kg;
+        if (kt < ntile) publish_max();
+        __syncthreads();  // the Q rows, or the last tile's fragments, are read
+        int ke = 0, ven = ve;
+        if (kt < ntile) {
+            const float mk = fmaxf(sh.am[kg][0][0], sh.am[kg][1][0]);
+            const float mv = fmaxf(sh.am[kg][0][1], sh.am[kg][1][1]);
+            const bool ok = split_range(mk) && split_range(mv);
+            fine = fine && ok;
+            ke = __builtin_amdgcn_readfirstlane(ok ? split_exp(mk) : 0);
+            ven = __builtin_amdgcn_readfirstlane(ok ? split_exp(mv) : 0);
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                uint4 p[2];
+                split2x8(kr[s], pow2i(ke), p[0], p[1]);
+#pragma unroll
+                for (int u = 0; u < 2; u++) sh.k[kg][((qb * KS + s) * 2 + u) * 64 + lane] = p[u];
+            }
+#pragma unroll
+            for (int j = 0; j < VD; j++) {
+                const float v[8] = {vr[0][j], vr[1][j], vr[2][j], vr[3][j],
+                                    vr[4][j], vr[5][j], vr[6][j], vr[7][j]};
+                uint4 p[2];
+                split2x8(v, pow2i(ven), p[0], p[1]);
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    sh.v[kg][((VD * (dg & 1) + j) * 2 + u) * 64 + vg * 16 + (dg >> 1)] = p[u];
+            }
+        }
+        __syncthreads();
+        if (kt + NG < ntile) load();  // in flight during this tile
+        if (kt >= ntile || !wave_rows || kPfSpKeys * kt > wave_hi) continue;
+
+        // S^T: [key tile][query tile]
+        v4f_t s[2][2];
+#pragma unroll
+        for (int k2 = 0; k2 < 2; k2++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) s[k2][j] = zero;
+#pragma unroll
+        for (int st = 0; st < KS; st++)
+#pragma unroll
+            for (int k2 = 0; k2 < 2; k2++) {
+                const uint4* f = sh.k[kg] + ((k2 * KS + st) * 2) * 64 + lane;
+                const uint4 kh = f[0], kl = f[64];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    s[k2][j] = mfma_h(kl, qp[j][st][0], s[k2][j]);
+                    s[k2][j] = mfma_h(kh, qp[j][st][1], s[k2][j]);
+                    s[k2][j] = mfma_h(kh, qp[j][st][0], s[k2][j]);
+                }
+            }
+        // online softmax of query col over its 8 keys of this lane
+        const bool diag = kPfSpKeys * kt + kPfSpKeys - 1 > wave_lo;
+        const float ck = c * pow2i(-ke);
+        const float dv = pow2i(ven - ve);
+        ve = ven;
+        float alpha[2];
+        uint4 pp[2][2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            float sv[8], tmax = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                sv[e] = s[e >> 2][j][e & 3];
+                if (diag && kPfSpKeys * kt + 16 * (e >> 2) + 4 * grp + (e & 3) > qpos[j])
+                    sv[e] = -INFINITY;
+                tmax = fmaxf(tmax, sv[e]);
+            }
+            const float Mn = fmaxf(M[j], ceilf(max_over_groups(tmax) * ck));
+            // a row with nothing to attend to yet keeps zero weights
+            const float Mr = Mn == -INFINITY ? 0.f : Mn - 14.f;  // p in units of 2^-14
+            alpha[j] = Mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(M[j] - Mn);
+            M[j] = Mn;
+            float ps = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                sv[e] = __builtin_amdgcn_exp2f(fmaf(sv[e], ck, -Mr));
+                ps += sv[e];
+            }
+            l[j] = fmaf(l[j], alpha[j], ps);
+            alpha[j] *= dv;
+            split2x8(sv, 1.f, pp[j][0], pp[j][1]);
+        }
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            const uint4* f = sh.v[kg] + t * 2 * 64 + lane;
+            const uint4 vh = f[0], vl = f[64];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                v4f_t x = mfma_h(vl, pp[j][0], zero);
+                x = mfma_h(vh, pp[j][1], x);
+                x = mfma_h(vh, pp[j][0], x);
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[j][t][r] = fmaf(o[j][t][r], alpha[j], x[r]);
+            }
+        }
+    }
+    if (!fine) sh.redo = 1;
+    if (lane == 0) sh.ve[kg][qb] = ve;
+    __syncthreads();
+
+    // 2. merge the key groups (the fragments are no longer read)
+    if (sh.redo) {
+        __syncthreads();
+        if (wave >= kPfKsWaves) return;  // ended waves take no part in barriers
+        // within k_attn_prefill_ks's token groups, so that a masked key's NaN (0 * inf)
+        // reaches no row that it does not reach there
+        const int qt16 = kPfKsRows / G, t_end = min(qt0 + QT, n_tok);
+        for (int t = qt0, nt; t < t_end; t += nt) {
+            nt = min(qt16 - t % qt16, t_end - t);
+            prefill_rows16<HD, false>(a, G, nt, kvh, t, sh.ks);
+            __syncthreads();
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int row = 32 * qb + 16 * j + col;
+        float* ow = sh.o + (kg * R + row) * QS + 4 * DT * grp;  // dims DT*(4*grp + r) + t
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t4 = 0; t4 < DT / 4; t4++)
+                *reinterpret_cast<float4*>(ow + r * DT + 4 * t4) = make_float4(
+                    o[j][4 * t4][r], o[j][4 * t4 + 1][r], o[j][4 * t4 + 2][r], o[j][4 * t4 + 3][r]);
+        l[j] += __shfl_xor(l[j], 16, 64);
+        l[j] += __shfl_xor(l[j], 32, 64);
+        if (grp == 0) {
+            sh.mm[kg][row] = M[j];
+            sh.ll[kg][row] = l[j];
+        }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < R * HD / 4; idx += kPfSpThreads) {
+        const int r = idx / (HD / 4), c4 = idx % (HD / 4), tl = r / G;
+        float Mx = sh.mm[0][r];
+#pragma unroll
+        for (int w = 1; w < NG; w++) Mx = fmaxf(Mx, sh.mm[w][r]);
+        float L = 0.f;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < NG; w++) {
+            const float f = sh.mm[w][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sh.mm[w][r] - Mx);
+            L = fmaf(sh.ll[w][r], f, L);
+            v = fma4(f * pow2i(-sh.ve[w][r >> 5]),
+                     *reinterpret_cast<const float4*>(sh.o + (w * R + r) * QS + 4 * c4), v);
+        }
+        const float inv = L > 0.f ? 1.f / L : 0.f;
+        v = make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);
+        if (tl < QT && qt0 + tl < n_tok)
+            store_out4<HD>(a, qt0 + tl, kvh * G + r % G, c4, v);
+    }
+}
+
 int attn_nsplit(int max_seq) { return (max_seq + kAttnSplit - 1) / kAttnSplit; }
 
 template <int HD>
 static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
     const int nt = a.n_tok > 1 ? a.n_tok : 1;
     if constexpr (HD <= 128) {
+        if constexpr (HD == 128) {
+            // the split products where 64-row workgroups nearly fill the chip and walk
+            // enough keys to pay for setting up (32 heads, 512 tokens, position 0:
+            // 44 us there, 48 here; from about position 300 on this one is faster).
+            // With 128 of them, or at head dimension 64, the 16-row kernel is ahead
+            // (16/2 heads, 512 tokens on 2000 keys: 126 and 166 us).
+            const int QS = kPfSpRows / G;
+            const dim3 gs((unsigned)a.n_kv_heads, (unsigned)((nt + QS - 1) / QS));
+            if (gs.x * gs.y >= 192 && !a.pos_dev && a.pos + nt / 2 >= 640) {
+                hipLaunchKernelGGL((k_attn_prefill_sp<HD>), gs, dim3(kPfSpThreads), 0, st, a, G, QS);
+                return hipGetLastError();
+            }
+        }
         const int QT = kPfKsRows / G;
         const dim3 grid((unsigned)a.n_kv_heads, (unsigned)((nt + QT - 1) / QT));
         // head dimension 128: prefetch registers leave two waves per SIMD instead of

@@ -1,0 +1,93 @@
+"""Prefill attention by split fp16 products (64-row workgroups) at its edges:
+group sizes that do not divide 64, ragged tokens, K and V of any scale, and
+values its scales do not cover, which take the fp32 kernel's arithmetic."""
+import numpy as np
+import pytest
+
+from llm_core_amd._ffi import call
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def attend(ctx, q, kc, vc, pos0, H, KVH, hd, cos_t, sin_t, path=0):
+    T = q.shape[0]
+    bufs = [ctx.upload(x) for x in (q, kc, vc, cos_t, sin_t)]
+    do, dq8 = ctx.alloc(T * H * hd * 4), ctx.alloc(T * H * hd // 32 * 36)
+    ctx.write(do, np.full(T * H * hd, 7e7, np.float32))
+    call("axf_hip_attn_prefill", ctx.handle, do.ptr, dq8.ptr, bufs[0].ptr, H * hd, None, bufs[1].ptr,
+         bufs[2].ptr, pos0, T, H, KVH, hd, bufs[3].ptr, bufs[4].ptr, path)
+    got = ctx.download(do, np.float32, T * H * hd).reshape(T, H * hd)
+    q8 = ctx.download(dq8, np.uint8, T * H * hd // 32 * 36).reshape(T, -1)
+    for b in bufs + [do, dq8]:
+        b.free()
+    return got, q8
+
+
+@pytest.mark.parametrize("H,KVH,T,pos0,kscale,vscale", [
+    (24, 24, 512, 384, 1.0, 1.0),     # exactly 192 workgroups, mean position 640
+    (28, 4, 440, 500, 1.0, 1.0),      # 7 heads per kv head: 9 tokens (63 rows), the last group ragged
+    (64, 8, 190, 700, 1.0, 1.0),      # 8 heads per kv head, 8 tokens per workgroup
+    (40, 40, 300, 1000, 3e-5, 1e9),   # small K (uniform weights), large V
+    (40, 40, 300, 1000, 40.0, 1e-8),  # one key takes nearly all of each row
+])
+def test_split_products_match_oracle(ctx, H, KVH, T, pos0, kscale, vscale):
+    hd, n = 128, pos0 + T
+    rng = np.random.default_rng(H + T)
+    q = rng.standard_normal((T, H * hd)).astype(np.float32)
+    kc = (rng.standard_normal(n * KVH * hd) * kscale).astype(np.float32)
+    vc = (rng.standard_normal(n * KVH * hd) * vscale).astype(np.float32)
+    cos_t, sin_t = O.rope_table(hd, 10000.0, n)
+    got, q8 = attend(ctx, q, kc, vc, pos0, H, KVH, hd, cos_t, sin_t)
+    k64, v64 = kc.reshape(n, KVH, hd).astype(np.float64), vc.reshape(n, KVH, hd).astype(np.float64)
+    for t in (0, 1, 8, 9, 63, T // 2, T - 2, T - 1):
+        qt = O.rope(q[t], pos0 + t, H, hd, cos_t, sin_t).reshape(H, hd).astype(np.float64)
+        seen = pos0 + t + 1
+        for h in range(0, H, 5):
+            k, v = k64[:seen, h // (H // KVH)], v64[:seen, h // (H // KVH)]
+            s = k @ qt[h] / np.sqrt(hd)
+            w = np.exp(s - s.max())
+            w /= w.sum()
+            err = np.abs(got[t, h * hd:(h + 1) * hd] - w @ v)
+            # a score carries 2^-22 of |q||k| / sqrt(hd) at most (split products and fp32
+            # sums), the weighted sum a few roundings of sum w |v|
+            smax = np.linalg.norm(qt[h]) * np.linalg.norm(k, axis=1).max() / np.sqrt(hd)
+            tol = (32 * 2.0 ** -24 + 2.0 ** -22 * smax) * (w @ np.abs(v))
+            assert (err <= tol).all(), (t, h, float((err / tol).max()))
+        assert np.array_equal(q8[t], O.quantize_q8_0(got[t]))
+
+
+def test_split_products_out_of_range(ctx):
+    """Infinities, NaN and magnitudes past 2^40: the rows that see them as the fp32
+    kernels leave them, the others as ever."""
+    H = KVH = 32
+    hd, T, pos0 = 128, 512, 512
+    n = pos0 + T
+    rng = np.random.default_rng(8)
+    q = rng.standard_normal((T, H * hd)).astype(np.float32)
+    kc = rng.standard_normal((n, KVH, hd)).astype(np.float32)
+    vc = rng.standard_normal((n, KVH, hd)).astype(np.float32)
+    kc[600, 3] *= 1e15
+    vc[700, 4, 5] = np.inf
+    vc[800, 5, 6] = np.nan
+    vc[:, 6] *= 1e-30
+    kc[900, 7] = -np.inf
+    cos_t, sin_t = O.rope_table(hd, 10000.0, n)
+    got, _ = attend(ctx, q, kc.ravel(), vc.ravel(), pos0, H, KVH, hd, cos_t, sin_t)
+    ref, _ = attend(ctx, q, kc.ravel(), vc.ravel(), pos0, H, KVH, hd, cos_t, sin_t, path=1)
+    got, ref = got.reshape(T, H, hd), ref.reshape(T, H, hd)
+    # what the fp32 kernels leave finite stays finite and equal
+    for h in range(H):
+        fine = np.isfinite(ref[:, h])
+        scale = np.abs(ref[:, h][fine]).max()
+        if h not in (4, 5, 7):
+            assert fine.all()
+        keep = fine & np.isfinite(got[:, h])
+        assert np.max(np.abs(got[:, h][keep] - ref[:, h][keep])) <= 1e-5 * scale, h
+        if h not in (4, 5, 7):
+            assert np.isfinite(got[:, h]).all(), h
+    # the fp32 kernel sums 16 tokens together (0 * inf of a masked key within them):
+    # the groups before the bad key's never see it
+    assert np.isfinite(got[: (700 - pos0) // 16 * 16, 4]).all()
+    assert np.isfinite(got[: (800 - pos0) // 16 * 16, 5]).all()
+    assert np.isfinite(got[: (900 - pos0) // 16 * 16, 7]).all()
