@@ -496,10 +496,15 @@ constexpr int kMiscMfmaMinT = 16;  // tokens from which the matrix-core form run
 
 // The A operand of k_gemm_misc_mfma, once per activation: token row t is
 // scaled by 2^E_t (max|x_t| * 2^E_t < 2^14, E_t in [-126, 126]) and each group
-// of 8 values u = 4b + g (block b, k-group g) stored as 8 fp16 hi then 8 fp16
-// lo at xhl[(u * T + t) * 32 bytes]; inv[t] = 2^-E_t.  A workgroup takes 4
-// tokens: each wave finds one row's maximum, then the 256 threads convert
-// with the token fastest (128 contiguous bytes per group).
+// of 8 values u = 4b + g (block b, k-group g) stored as 8 fp16 hi at
+// xhl[(2u * T + t) * 16 bytes] and 8 fp16 lo at xhl[((2u + 1) * T + t) * 16], so
+// that the GEMM's loads of 16 tokens are 256 contiguous bytes each (32 bytes of
+// hi and lo per token cost it two half-used loads); inv[t] = 2^-E_t.  A
+// workgroup takes 4 tokens and a share of the groups (gridDim.y): each wave
+// finds one row's maximum, then the 256 threads convert with the token fastest.
+// Up to 128 tokens, or for long rows, 4 workgroups share a row's groups (4096 x
+// 4096, 64 tokens: Q8_0 32.3 -> 29.8 us with both, F16 28.7 -> 26.8); at 200 x
+// 896 finding each maximum four times costs more (25.8 and 26.1 us).
 __global__ __launch_bounds__(256) void k_prep_hl_rows(const float* __restrict__ X, int cols, int T,
                                                       uint8_t* __restrict__ xhl,
                                                       float* __restrict__ inv) {
@@ -522,7 +527,7 @@ __global__ __launch_bounds__(256) void k_prep_hl_rows(const float* __restrict__ 
         const int E = max(min(140 - (int)(m >> 23), 126), -126);
         if (lane == 0) {
             scl[wave] = __uint_as_float((uint32_t)(E + 127) << 23);
-            if (t < T) inv[t] = __uint_as_float((uint32_t)(127 - E) << 23);
+            if (t < T && blockIdx.y == 0) inv[t] = __uint_as_float((uint32_t)(127 - E) << 23);
         }
     }
     __syncthreads();
@@ -530,7 +535,7 @@ __global__ __launch_bounds__(256) void k_prep_hl_rows(const float* __restrict__ 
     if (t >= T) return;
     const float sc = scl[tt];
     const float* xr = X + (size_t)t * cols;
-    for (int u = threadIdx.x >> 2; u < cols / 8; u += 64) {
+    for (int u = blockIdx.y * 64 + (threadIdx.x >> 2); u < cols / 8; u += 64 * gridDim.y) {
         const float4 a = reinterpret_cast<const float4*>(xr + 8 * u)[0];
         const float4 b = reinterpret_cast<const float4*>(xr + 8 * u)[1];
         float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -545,9 +550,9 @@ __global__ __launch_bounds__(256) void k_prep_hl_rows(const float* __restrict__ 
             hi[e] = h;
             lo[e] = (_Float16)(xs - (float)h);
         }
-        uint8_t* p = xhl + ((size_t)u * T + t) * 32;
+        uint8_t* p = xhl + ((size_t)(2 * u) * T + t) * 16;
         *reinterpret_cast<mh8_t*>(p) = hi;
-        *reinterpret_cast<mh8_t*>(p + 16) = lo;
+        *reinterpret_cast<mh8_t*>(p + (size_t)T * 16) = lo;
     }
 }
 
@@ -625,6 +630,39 @@ __device__ __forceinline__ mh8_t misc_decode(const MiscRaw& r, int g, float& d) 
     }
 }
 
+// A result lane's NJ tiles: tokens t + 16j + 0..3 of row o, scaled by inv.  All
+// scales (and old values) are loaded before the first store, not one by one
+// behind the bounds checks (Q8_0 896 x 896, 200 tokens: 12.7 -> 11.5 us).
+template <int NJ>
+__device__ __forceinline__ void misc_store(float* __restrict__ Y, const float* __restrict__ inv,
+                                           const mf4_t (&acc)[NJ], long o, int rows, int t, int T,
+                                           int accumulate) {
+    float s[NJ][4], v[NJ][4];
+    const long oc = min(o, (long)rows - 1);
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) s[j][q] = inv[min(t + 16 * j + q, T - 1)];
+    if (accumulate) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[j][q] = Y[(size_t)min(t + 16 * j + q, T - 1) * rows + oc];
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float r = acc[j][q] * s[j][q];
+            v[j][q] = accumulate ? v[j][q] + r : r;
+        }
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (o < rows && t + 16 * j + q < T) Y[(size_t)(t + 16 * j + q) * rows + o] = v[j][q];
+}
+
 // KS waves of a workgroup split K (contiguous block ranges, partial tiles added
 // in wave order through LDS) and kMmWaves / KS waves take consecutive row
 // groups; the block loop loads block b + 1 before computing block b.
@@ -645,11 +683,11 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 #pragma unroll
     for (int i = 0; i < kMmRTW; i++)
         wr[i] = W + min(row0 + 16 * i + col, (long)rows - 1) * row_bytes;  // past the end: not stored
-    const uint8_t* xr[kMmTTW];  // this lane's token: group u = 4b + g at xr + u*T*32
+    const uint8_t* xr[kMmTTW];  // this lane's token: group u = 4b + g's hi at xr + 4b*T*32
 #pragma unroll
     for (int j = 0; j < kMmTTW; j++) {
         const int t = min(t0 + 16 * j + col, T - 1);  // past T: not stored
-        xr[j] = xhl + ((size_t)g * T + t) * 32;
+        xr[j] = xhl + ((size_t)(2 * g) * T + t) * 16;
     }
     const mf4_t zero = {0.f, 0.f, 0.f, 0.f};
     mf4_t acc[kMmRTW][kMmTTW];
@@ -669,7 +707,7 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
         for (int j = 0; j < kMmTTW; j++) {
             const uint8_t* p = xr[j] + (size_t)bb * 4 * T * 32;
             xh[j] = *reinterpret_cast<const mh8_t*>(p);
-            xl[j] = *reinterpret_cast<const mh8_t*>(p + 16);
+            xl[j] = *reinterpret_cast<const mh8_t*>(p + (size_t)T * 16);
         }
     };
     if (b0 < b1) load(b0);
@@ -717,20 +755,176 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
                 for (int j = 0; j < kMmTTW; j++) acc[i][j] += part[q][rg][i * kMmTTW + j][lane];
     }
 #pragma unroll
-    for (int i = 0; i < kMmRTW; i++) {
-        const long o = row0 + 16 * i + col;
+    for (int i = 0; i < kMmRTW; i++)
+        misc_store<kMmTTW>(Y, inv, acc[i], row0 + 16 * i + col, rows, t0 + 4 * g, T, accumulate);
+}
+
+// The same product with a token group's activations shared through LDS: a
+// workgroup owns 64 rows x 64 tokens, 4 row groups of 16 x 2 K ranges (8 waves).
+// In k_gemm_misc_mfma every 16-row wave reads its tokens' hi/lo rows from L2 by
+// itself (4864 x 896, 200 tokens: 279 MB, and 7 scattered loads per Q5_0 block),
+// which bounds it.  Here the four row groups share each 2-block stage (16 KB,
+// loaded into registers during the stage before), and a wave's two blocks
+// per row come as 12 (Q5_0) or 20 (Q8_0) dwords, 3 or 5 coalesced loads instead
+// of 14 or 8, spread to the lanes through LDS.  Sums are kept per quarter of K,
+// as with 4 K ranges there.
+// Whole calls before and now, Q5_0 / Q8_0 / F16: 4864 x 896, 512 tokens 49 -> 34,
+// 45 -> 36, 38 -> 29 us; 11008 x 4096, 128 tokens 143 -> 76, 123 -> 98, 93 -> 60 us;
+// 4864 x 896, 200 tokens 28.5 -> 23.9, 26 -> 25, 22 -> 18 us.  Each stage waits for
+// the next one's loads; bringing the first lines into L2 ahead of the loop was
+// slower (25.6 us for 23.9).
+constexpr int kMsWaves = 8, kMsTok = 64, kMsRows = 64;
+
+template <int QT>
+__global__ __launch_bounds__(kMsWaves * 64, 4) void k_gemm_misc_shared(
+    float* __restrict__ Y, const uint8_t* __restrict__ W, const uint8_t* __restrict__ xhl,
+    const float* __restrict__ inv, int rows, int cols, long row_bytes, int T, int accumulate) {
+    constexpr int NJ = kMsTok / 16;
+    __shared__ mu4_t xs[2][2][16][kMsTok];  // [K range][buffer][8 block + 2 k-group + lo][token]
+    constexpr uint32_t BS = QT == 8 ? 34 : 22;  // bytes of a block
+    constexpr int ND = QT == 8 ? 20 : 12;       // dwords kept of two blocks: 18 and 12 hold them
+    __shared__ uint32_t ws[QT == 1 ? 1 : kMsWaves][16][ND];
+    const int tid = threadIdx.x, lane = tid & 63, st = tid & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave >> 2, rg = wave & 3;
+    const int col = lane & 15, g = lane >> 4;
+    const long row0 = (long)blockIdx.x * kMsRows + 16 * rg;
+    const int t0 = blockIdx.y * kMsTok;
+    const int nb = cols / 32, np = (nb + 1) / 2, h = (np + 1) / 2;
+    const int p0 = ks * h, p1 = min(np, p0 + h);  // this K range, in pairs of blocks
+    const uint8_t* wr = W + min(row0 + col, (long)rows - 1) * row_bytes;  // past the end: not stored
+    // activation pieces of this thread: fragments st / 64 + 4i, token st % 64, as byte
+    // offsets (a last odd block's second half: valid rows, unused)
+    const uint32_t xt = (uint32_t)min(t0 + (st & 63), T - 1) * 16;  // past T: not stored
+    const uint32_t xstep = (uint32_t)T * 16, xlast = (uint32_t)(8 * nb - 1) * xstep + xt;
+    // the row's dwords from the one that holds its first byte
+    const uint32_t w0 = QT == 1 ? 0 : (uint32_t)(reinterpret_cast<uintptr_t>(wr) & 3u);
+    const uint8_t* wa = wr - w0;
+    const uint32_t wlast = (w0 + BS * (uint32_t)nb - 1) & ~3u;
+    mu4_t xr[4];
+    MiscRaw raw[2];
+    uint32_t wd[ND / 4];
+    auto load = [&](int p) {
+        uint32_t xo = (16u * p + (st >> 6)) * xstep + xt;
 #pragma unroll
-        for (int j = 0; j < kMmTTW; j++)
+        for (int i = 0; i < 4; i++, xo += 4 * xstep)
+            xr[i] = *reinterpret_cast<const mu4_t*>(xhl + min(xo, xlast));
+        if constexpr (QT == 1) {
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++) {
-                const int t = t0 + 16 * j + 4 * g + ii;
-                if (o < rows && t < T) {
-                    const float v = acc[i][j][ii] * inv[t];
-                    float* y = Y + (size_t)t * rows + o;
-                    *y = accumulate ? *y + v : v;
-                }
-            }
+            for (int k = 0; k < 2; k++) misc_load<QT>(wr, min(2 * p + k, nb - 1), g, raw[k]);
+        } else {
+            // dwords g, g + 4, ... of the two blocks, none past the one that holds the
+            // row's last byte
+            const uint32_t o = ((w0 + 2u * BS * p) & ~3u) + 4u * g;
+#pragma unroll
+            for (int i = 0; i < ND / 4; i++)
+                wd[i] = *reinterpret_cast<const uint32_t*>(wa + min(o + 16u * i, wlast));
+        }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) xs[ks][buf][(st >> 6) + 4 * i][st & 63] = xr[i];
+    };
+    const mf4_t zero = {0.f, 0.f, 0.f, 0.f};
+    mf4_t acc[NJ], held[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[j] = held[j] = zero;
+    if (p0 < p1) {
+        load(p0);
+        put(0);
     }
+    __syncthreads();
+#pragma unroll 1
+    for (int i = 0, ie = (h + 1) / 2; i < h; ie = h) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            held[j] = acc[j];
+            acc[j] = zero;
+        }
+#pragma unroll 1
+        for (; i < ie; i++) {  // the same count, and barriers, in every wave
+            const int p = p0 + i;
+            if (p < p1) {
+                mh8_t bw[2];
+                float d[2];
+                if constexpr (QT == 1) {
+#pragma unroll
+                    for (int k = 0; k < 2; k++) bw[k] = misc_decode<QT>(raw[k], g, d[k]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < ND / 4; k++) ws[wave][col][g + 4 * k] = wd[k];
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    const uint32_t* w = ws[wave][col];
+                    const uint32_t s0 = (w0 + 2u * BS * p) & 3u;
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {  // as misc_load; the block starts at byte o of w
+                        const uint32_t o = s0 + BS * k, hs = 8 * (o & 3u);
+                        MiscRaw cur;
+                        cur.sh = o & 3u;
+                        cur.d = (w[o / 4] >> hs) & 0xffffu;
+                        if constexpr (QT == 8) {
+                            cur.w[0] = w[(o + 2) / 4 + 2 * g];
+                            cur.w[1] = w[(o + 2) / 4 + 2 * g + 1];
+                            cur.w[2] = (w[(o + 8) / 4 + 2 * g] >> hs) & 0xffffu;
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 5; q++) cur.w[q] = w[(o + 2) / 4 + q];
+                            cur.w[5] = (w[(o + 20) / 4] >> hs) & 0xffffu;
+                        }
+                        bw[k] = misc_decode<QT>(cur, g, d[k]);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+                if (p + 1 < p1) load(p + 1);  // in flight during this pair's products
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    if (2 * p + k >= nb) break;
+                    // every fragment is read before the first product (left alone, the
+                    // compiler waited for each tile's pair in turn)
+                    mh8_t ah[NJ], al[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        ah[j] = __builtin_bit_cast(mh8_t, xs[ks][i & 1][8 * k + 2 * g][16 * j + col]);
+                        al[j] = __builtin_bit_cast(mh8_t, xs[ks][i & 1][8 * k + 2 * g + 1][16 * j + col]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    mf4_t c[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+                        c[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], bw[k], QT == 1 ? acc[j] : zero, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+                        c[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[j], bw[k], c[j], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        if constexpr (QT == 1) {
+                            acc[j] = c[j];
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 4; q++) acc[j][q] = fmaf(d[k], c[j][q], acc[j][q]);
+                        }
+                    }
+                }
+                if (p + 1 < p1) put((i + 1) & 1);
+            }
+            __syncthreads();
+        }
+    }
+    // K range 1's tiles through LDS (the stages are no longer read)
+    mf4_t* part = reinterpret_cast<mf4_t*>(&xs[0][0][0][0]);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        acc[j] = held[j] + acc[j];
+        if (ks) part[(rg * NJ + j) * 64 + lane] = acc[j];
+    }
+    __syncthreads();
+    if (ks) return;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[j] += part[(rg * NJ + j) * 64 + lane];
+    misc_store<NJ>(Y, inv, acc, row0 + col, rows, t0 + 4 * g, T, accumulate);
 }
 
 template <int TT, int KS>
@@ -771,9 +965,30 @@ hipError_t launch_gemm_misc_f32(int qtype, float* Y, const void* W, const float*
     if (scratch && gemm_misc_mfma_applies(T, X)) {
         float* iv = scratch;
         auto* xhl = reinterpret_cast<uint8_t*>(scratch + (T + 3) / 4 * 4);  // 16-byte aligned
+        const unsigned prep_y = T <= 128 || (T < 1024 && cols >= 2048) ? 4 : 1;
         if (!prepared)
-            hipLaunchKernelGGL(k_prep_hl_rows, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, X,
+            hipLaunchKernelGGL(k_prep_hl_rows, dim3((unsigned)((T + 3) / 4), prep_y), dim3(256), 0, st, X,
                                cols, T, xhl, iv);
+        const int bs = qtype == 8 ? 34 : 22;
+        const dim3 gs((unsigned)((rows + kMsRows - 1) / kMsRows), (unsigned)((T + kMsTok - 1) / kMsTok));
+        // whole dwords of Q8_0 and Q5_0 rows lie inside W where it starts and ends on one
+        const bool dwords = qtype == 1 || (((reinterpret_cast<uintptr_t>(w8) & 3) == 0) &&
+                                           ((rows - 1) * row_bytes + cols / 32 * (long)bs) % 4 == 0 &&
+                                           row_bytes % 2 == 0);
+        // The shared form from 160 workgroups (2560 x 4096, 200 tokens: Q5_0 79 -> 55 us,
+        // Q8_0 69 -> 61, F16 51 -> 49); with 128 (2048 x 896, 200 tokens) it took 17.1, 17.3
+        // and 15.1 us against 16.8, 16.2 and 14.6, with fewer it is far behind.  Its offsets
+        // are 32-bit.
+        if (T > 32 && dwords && (long)gs.x * gs.y >= 160 && (size_t)T * cols * 4 < (1u << 31) &&
+            cols / 32 * (long)bs < (1l << 31)) {
+            if (qtype == 1)
+                hipLaunchKernelGGL((k_gemm_misc_shared<1>), gs, dim3(kMsWaves * 64), 0, st, Y, w8, xhl, iv, rows, cols, row_bytes, T, accumulate);
+            else if (qtype == 8)
+                hipLaunchKernelGGL((k_gemm_misc_shared<8>), gs, dim3(kMsWaves * 64), 0, st, Y, w8, xhl, iv, rows, cols, row_bytes, T, accumulate);
+            else
+                hipLaunchKernelGGL((k_gemm_misc_shared<6>), gs, dim3(kMsWaves * 64), 0, st, Y, w8, xhl, iv, rows, cols, row_bytes, T, accumulate);
+            return hipGetLastError();
+        }
         // K split over the workgroup's waves where the row groups x token groups
         // leave fewer than 2048 workgroups (K ranges of at least 4 blocks)
         const long tg = (T + 16 * kMmTTW - 1) / (16 * kMmTTW), nb = cols / 32;
