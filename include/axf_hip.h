@@ -191,7 +191,8 @@ typedef struct {
  * rep_penalty_last_n of hist[0..n_hist) (llama_model.cpp:1595-1605; applied to
  * logits_dev in place, as the reference does to state.logits), then sample()
  * (:1466-1498) with the uniform draw r.  *token (host) receives the id.  Any
- * top_k: up to 16384 candidates (ceil(n_vocab / 4096) * min(k, 4096)) are
+ * top_k: up to 64 candidates are selected by a threshold (penalty windows up to
+ * 1024 tokens); otherwise up to 16384 (ceil(n_vocab / 4096) * min(k, 4096)) are
  * sorted in LDS, more (e.g. top_k above 431 at n_vocab 151936, or the whole
  * vocabulary) in place in device memory by one workgroup, a few ms per call.
  * Among exactly equal scores the lower index ranks first. */

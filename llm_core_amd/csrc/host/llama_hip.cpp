@@ -101,12 +101,12 @@ struct axf_llama {
     // and of h's Q8_0 blocks, written by the gate|up GEMM's SwiGLU epilogue
     uint8_t* pf_hxh = nullptr;
     float *pf_hdx2 = nullptr, *pf_hgx2 = nullptr, *pf_hdx4 = nullptr;
-    // prefill attention: the matrix-core kernel, or (testing) the decode
+    // prefill attention: the matrix-core kernels, or (testing) the decode
     // split/combine kernels over a token grid
     bool pf_attn_split = false;
 
     // sampled generation (allocated on first use): penalty history (prompt and
-    // generated tokens) and its length, the step's uniform draws, sort keys
+    // generated tokens) and its length, the step's uniform draws, candidate keys
     int *d_hist = nullptr, *d_hist_n = nullptr;
     float* d_r = nullptr;
     uint64_t* d_cand = nullptr;

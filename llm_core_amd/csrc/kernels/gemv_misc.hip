@@ -479,9 +479,10 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_misc_f32(
 // Q8_0; F16 accumulates in the MFMA), and the result by 2^-E_t.  The sums
 // differ from the per-token GEMV's sequential fp32 sums in rounding only.
 // Tokens are A's rows and weight rows B's columns: a result lane holds tokens
-// 4g..4g+3 of one weight row, so d is the lane's own row's.  A wave owns RTW
-// row tiles x TTW token tiles (16 x 16 each); a workgroup 4 waves on
-// consecutive row tiles of one token group.
+// 4g..4g+3 of one weight row, so d is the lane's own row's.  In
+// k_gemm_misc_mfma a wave owns RTW row tiles x TTW token tiles (16 x 16 each);
+// a workgroup 4 waves on consecutive row tiles of one token group.
+// k_gemm_misc_shared (below) shares the activations of larger grids in LDS.
 // ---------------------------------------------------------------------------
 typedef _Float16 mh8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 mh2_t __attribute__((ext_vector_type(2)));
