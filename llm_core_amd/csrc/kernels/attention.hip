@@ -915,14 +915,18 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
 // 32 heads of 128, 512 tokens at position 1536: error against 64 bits 5.6e-7
 // with fp32 products, 3.4e-7 here; 183 -> 143 us (15 GFLOP, 105 TFLOP/s).
 //
-// The scales cover tiles whose largest |x| is in [2^-40, 2^40) or 0.  A
-// workgroup that meets another (infinities, say) computes its rows again with
-// k_attn_prefill_ks's arithmetic.
+// The scales cover tiles whose largest |x| is in [2^-40, 2^40) or 0, and the
+// exponent's one fma holds p within fp16 while |M| is small: max * c is rounded
+// before M's ceiling is taken, the fma's product is not, and the difference is
+// 2^-24 |M| (from 2^24 on p can pass 65504, or vanish for every key).  A
+// workgroup that meets a tile outside the scales (infinities, say) or ends with
+// |M| > 2^20 computes its rows again with k_attn_prefill_ks's arithmetic.
 // ---------------------------------------------------------------------------
 constexpr int kPfSpRows = 64;    // query rows per workgroup
 constexpr int kPfSpKeys = 32;    // keys per tile
 constexpr int kPfSpGroups = 4;   // key groups
 constexpr int kPfSpThreads = kPfSpGroups * 128;
+constexpr float kPfSpMaxM = 0x1p20f;  // p <= 2^14 * 2^(2^-4) up to here
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
@@ -1235,6 +1239,9 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
             }
         }
     }
+    // the final M decides: an earlier one far below it left weights of 2^(M_old - M) = 0
+#pragma unroll
+    for (int j = 0; j < 2; j++) fine = fine && (M[j] == -INFINITY || fabsf(M[j]) <= kPfSpMaxM);
     if (!fine) sh.redo = 1;
     if (lane == 0) sh.ve[kg][qb] = ve;
     __syncthreads();

@@ -91,3 +91,39 @@ def test_split_products_out_of_range(ctx):
     assert np.isfinite(got[: (700 - pos0) // 16 * 16, 4]).all()
     assert np.isfinite(got[: (800 - pos0) // 16 * 16, 5]).all()
     assert np.isfinite(got[: (900 - pos0) // 16 * 16, 7]).all()
+
+
+@pytest.mark.parametrize("H,KVH,std", [
+    (32, 32, 1e3), (32, 32, 3e3), (32, 32, 6e3), (32, 32, 2e4), (128, 16, 5e4), (32, 32, 1e6),
+])
+def test_split_products_large_scores(ctx, H, KVH, std):
+    """q.k / sqrt(hd) from 1e6 to 1e12 with every operand well inside the scales: the
+    softmax is one key's, and the row that key's V."""
+    hd, T, pos0 = 128, 512, 512
+    n, G = pos0 + T, H // KVH
+    rng = np.random.default_rng(int(std))
+    q = (rng.standard_normal((T, H * hd)) * std).astype(np.float32)
+    kc = (rng.standard_normal((n, KVH, hd)) * std).astype(np.float32)
+    vc = rng.standard_normal((n, KVH, hd)).astype(np.float32)
+    cos_t, sin_t = O.rope_table(hd, 10000.0, n)
+    got, _ = attend(ctx, q, kc.ravel(), vc.ravel(), pos0, H, KVH, hd, cos_t, sin_t)
+    assert np.isfinite(got).all()
+    got = got.reshape(T, H, hd)
+    clear = 0
+    for t in range(0, T, 3):
+        qt = O.rope(q[t], pos0 + t, H, hd, cos_t, sin_t).reshape(H, hd).astype(np.float64)
+        seen = pos0 + t + 1
+        for h in (t % H, (7 * t + 5) % H):
+            k = kc[:seen, h // G].astype(np.float64)
+            s = k @ qt[h] / np.sqrt(hd)
+            best, second = np.argsort(s)[:-3:-1]
+            # a score's error: 128 fp32 products and sums, and the scaling's rounding
+            err = 2.0 ** -24 * 130 * np.linalg.norm(qt[h]) * np.linalg.norm(k, axis=1).max() / np.sqrt(hd)
+            # with the two best further apart than both errors and ln(seen * 2^24) the
+            # others' weights are under one rounding of the sum
+            if s[best] - s[second] < 2 * err + np.log(seen * 2.0 ** 24):
+                continue
+            clear += 1
+            v = vc[best, h // G]
+            assert np.abs(got[t, h] - v).max() <= 4 * 2.0 ** -24 * np.abs(v).max(), (t, h)
+    assert clear > 50
