@@ -919,8 +919,11 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
 // exponent's one fma holds p within fp16 while |M| is small: max * c is rounded
 // before M's ceiling is taken, the fma's product is not, and the difference is
 // 2^-24 |M| (from 2^24 on p can pass 65504, or vanish for every key).  A
-// workgroup that meets a tile outside the scales (infinities, say) or ends with
-// |M| > 2^20 computes its rows again with k_attn_prefill_ks's arithmetic.
+// workgroup that meets a tile outside the scales (infinities, say), ends with
+// |M| > 2^20 or with results that are no numbers computes its rows again with
+// k_attn_prefill_ks's arithmetic.  The last is how a NaN shows: the maxima drop
+// it, but 0 * NaN in the products carries a masked key's to every row of the
+// wave, and k_attn_prefill_ks's to its 16 only.
 // ---------------------------------------------------------------------------
 constexpr int kPfSpRows = 64;    // query rows per workgroup
 constexpr int kPfSpKeys = 32;    // keys per tile
@@ -1242,6 +1245,16 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
     // the final M decides: an earlier one far below it left weights of 2^(M_old - M) = 0
 #pragma unroll
     for (int j = 0; j < 2; j++) fine = fine && (M[j] == -INFINITY || fabsf(M[j]) <= kPfSpMaxM);
+    float zero_sum = 0.f;  // NaN if any result is not finite
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        zero_sum = fmaf(l[j], 0.f, zero_sum);
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) zero_sum = fmaf(o[j][t][r], 0.f, zero_sum);
+    }
+    fine = fine && zero_sum == 0.f;
     if (!fine) sh.redo = 1;
     if (lane == 0) sh.ve[kg][qb] = ve;
     __syncthreads();
