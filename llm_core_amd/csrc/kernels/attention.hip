@@ -1326,7 +1326,9 @@ static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
             // (16/2 heads, 512 tokens on 2000 keys: 126 and 166 us).
             const int QS = kPfSpRows / G;
             const dim3 gs((unsigned)a.n_kv_heads, (unsigned)((nt + QS - 1) / QS));
-            if (gs.x * gs.y >= 192 && !a.pos_dev && a.pos + nt / 2 >= 640) {
+            // its K and V row offsets are 32-bit, up to 160 rows past the last key
+            const bool offsets = ((uint64_t)a.pos + nt + 160) * a.n_kv_heads * HD * 4 <= UINT32_MAX;
+            if (gs.x * gs.y >= 192 && !a.pos_dev && a.pos + nt / 2 >= 640 && offsets) {
                 hipLaunchKernelGGL((k_attn_prefill_sp<HD>), gs, dim3(kPfSpThreads), 0, st, a, G, QS);
                 return hipGetLastError();
             }

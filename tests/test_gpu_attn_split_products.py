@@ -131,3 +131,42 @@ def test_split_products_large_scores(ctx, H, KVH, std):
             v = vc[best, h // G]
             assert np.abs(got[t, h] - v).max() <= 4 * 2.0 ** -24 * np.abs(v).max(), (t, h)
     assert clear > 50
+
+
+def test_cache_past_32_bit_offsets(ctx):
+    """A layer's K (and V) of over 4 GiB: 272 KV heads and nearly 32768 positions, rows
+    that repeat every 241 positions (no divisor of a wrapped offset's distance)."""
+    H, hd, T, pos0, period = 272, 128, 64, 32700, 241
+    n = pos0 + T
+    rng = np.random.default_rng(3)
+    kb, vb = (rng.standard_normal((period, H, hd), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((T, H * hd), dtype=np.float32)
+    row = H * hd * 4
+    caches = []
+    for b in (kb, vb):
+        c = ctx.alloc(n * row)
+        ctx.write(c, b)
+        for i in range(period, n, period):
+            ctx.copy(c.at(i * row), c, min(period, n - i) * row)
+        caches.append(c)
+    dq, cos, sin = (ctx.upload(x) for x in (q, np.ones((n, hd // 2), np.float32),
+                                            np.zeros((n, hd // 2), np.float32)))
+    do = ctx.upload(np.full(T * H * hd, np.nan, np.float32))
+    call("axf_hip_attn_prefill", ctx.handle, do.ptr, None, dq.ptr, H * hd, None, caches[0].ptr,
+         caches[1].ptr, pos0, T, H, H, hd, cos.ptr, sin.ptr, 0)
+    got = ctx.download(do, np.float32, T * H * hd).reshape(T, H, hd)
+    for b in caches + [dq, cos, sin, do]:
+        b.free()
+    for h in (0, 100, 271):
+        for t in (0, 40, T - 1):
+            seen = pos0 + t + 1
+            times = np.bincount(np.arange(seen) % period, minlength=period)
+            qt = q[t].reshape(H, hd)[h].astype(np.float64)
+            k, v = kb[:, h].astype(np.float64), vb[:, h].astype(np.float64)
+            s = k @ qt / np.sqrt(hd)
+            w = np.exp(s - s.max()) * times
+            w /= w.sum()
+            # as above, and the weights' sum of `seen` terms
+            smax = np.linalg.norm(qt) * np.linalg.norm(k, axis=1).max() / np.sqrt(hd)
+            tol = ((32 + seen / 64) * 2.0 ** -24 + 2.0 ** -22 * smax) * (w @ np.abs(v))
+            assert (np.abs(got[t, h] - w @ v) <= tol).all(), (t, h)
