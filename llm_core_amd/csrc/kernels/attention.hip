@@ -885,14 +885,22 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
 }
 
 // ---------------------------------------------------------------------------
-// The same attention on the fp16 matrix cores, fp32 kept by splitting: a tile's
-// values are scaled by a power of two so that the largest is in [2^14, 2^15)
-// and written as x = h + l, two fp16 parts rounded one after the other (22 bits
-// and the sign of l: 2^-23 of x, for values down to 2^-15 of the largest;
-// 2^-40 of the largest below).  A product is hh + hl + lh, accumulated in fp32,
-// the small ones first; ll is under 2^-24 of it.  v_mfma_f32_16x16x32_f16 does
-// 8x the products of v_mfma_f32_16x16x4_f32 in half its cycles, so three of
-// them cost 3/16.
+// The same attention on the fp16 matrix cores, fp32 kept by splitting: values
+// are scaled by a power of two so that the largest is in [2^14, 2^15), and
+// written as x = h + l, two fp16 parts rounded one after the other (22 bits and
+// the sign of l: 2^-23 of x).  A product is hh + hl + lh, accumulated in fp32;
+// ll is 2^-22 of it at most, 2^-25 in the mean square.  v_mfma_f32_16x16x32_f16 does 8x the products of
+// v_mfma_f32_16x16x4_f32 in half its cycles, so three of them cost 3/16.
+// fp16's smallest steps end the 22 bits for values far below the largest, so
+// what shares a scale is kept small or l is kept large:
+//   Q, K   a scale per row and per key: 2^-23 of a value down to 2^-16 of its
+//          row's largest, 2^-40 of the largest below (under 2^-35 |q||k| in a
+//          score);
+//   V      a scale per 32-key tile, the smallest so far, and l times 2^11 with
+//          sums of its own: 2^-23 down to 2^-27 of the tiles' largest, 2^-50 of
+//          it below, so that a value neither the row nor the channel uses (a
+//          later key's, another channel's) costs the others nothing;
+//   P      as V, in units of 2^-14.
 //
 // A workgroup owns 64 query rows of one kv head (QT = 64 / G tokens x the G
 // heads that share it): 4 key groups x 2 waves of 32 rows, two waves per SIMD.
@@ -911,19 +919,21 @@ __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a,
 //                holds DT consecutive dims.
 // The running maximum is kept as a whole power of two, M = ceil(max * log2(e)
 // / sqrt(HD)): p = 2^(s * c - M) is one fma and one v_exp_f32, and rescaling by
-// 2^(M_old - M_new) is exact, as are the tiles' scales.
-// 32 heads of 128, 512 tokens at position 1536: error against 64 bits 5.6e-7
-// with fp32 products, 3.4e-7 here; 183 -> 143 us (15 GFLOP, 105 TFLOP/s).
+// 2^(M_old - M_new) is exact, as are the scales.
+// 32 heads of 128, 512 tokens at position 1536 (15 GFLOP): 183 us with fp32
+// products, 137 here (110 TFLOP/s); error against 64 bits 5.6e-7 and 3.4e-7.
+// With one Q scale per 32 rows, one K scale per tile and l left small it took
+// 149 us, and a value 2^-30 of its tile's largest kept 3 digits.  Summing hh
+// straight into o takes 128 us, but its error is 3.6e-7.
 //
-// The scales cover tiles whose largest |x| is in [2^-40, 2^40) or 0, and the
-// exponent's one fma holds p within fp16 while |M| is small: max * c is rounded
-// before M's ceiling is taken, the fma's product is not, and the difference is
-// 2^-24 |M| (from 2^24 on p can pass 65504, or vanish for every key).  A
-// workgroup that meets a tile outside the scales (infinities, say), ends with
-// |M| > 2^20 or with results that are no numbers computes its rows again with
-// k_attn_prefill_ks's arithmetic.  The last is how a NaN shows: the maxima drop
-// it, but 0 * NaN in the products carries a masked key's to every row of the
-// wave, and k_attn_prefill_ks's to its 16 only.
+// The exponent's one fma holds p within fp16 while |M| is small: max * c is
+// rounded before M's ceiling is taken, the fma's product is not, and the
+// difference is 2^-24 |M| (from 2^24 on p can pass 65504, or vanish for every
+// key).  A workgroup that ends with |M| > 2^20 or with results that are not
+// finite computes its rows again with k_attn_prefill_ks's arithmetic.  The last
+// is how infinities and NaN show: the maxima drop a NaN, but 0 * NaN in the
+// products carries a masked key's to every row of the wave, and
+// k_attn_prefill_ks's to its 16 only.
 // ---------------------------------------------------------------------------
 constexpr int kPfSpRows = 64;    // query rows per workgroup
 constexpr int kPfSpKeys = 32;    // keys per tile
@@ -934,28 +944,27 @@ constexpr float kPfSpMaxM = 0x1p20f;  // p <= 2^14 * 2^(2^-4) up to here
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 
-// x * s for 8 floats as two 8-element operands h + l
+// x * s for 8 floats as two 8-element operands h + l / LS
+template <int LS>
 __device__ __forceinline__ void split2x8(const float (&x)[8], float s, uint4& h, uint4& l) {
     uint32_t ph[4], pl[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const float a = x[2 * i], b = x[2 * i + 1];
         const h2_t hh = {(_Float16)(a * s), (_Float16)(b * s)};
-        const h2_t lo = {(_Float16)fmaf(a, s, -(float)hh.x), (_Float16)fmaf(b, s, -(float)hh.y)};
+        const h2_t lo = {(_Float16)((float)LS * fmaf(a, s, -(float)hh.x)),
+                         (_Float16)((float)LS * fmaf(b, s, -(float)hh.y))};
         ph[i] = __builtin_bit_cast(uint32_t, hh);
         pl[i] = __builtin_bit_cast(uint32_t, lo);
     }
     h = make_uint4(ph[0], ph[1], ph[2], ph[3]);
     l = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 }
+constexpr int kPfSpLow = 2048;  // LS of P and V
 
-__device__ __forceinline__ bool split_range(float amax) {
-    return amax == 0.f || (amax >= 0x1p-40f && amax < 0x1p40f);
-}
-
-// e with amax * 2^e in [2^14, 2^15) (0 for amax = 0), for amax in split_range
+// e with amax * 2^e in [2^14, 2^15), at most 126 (amax under 2^-112, or 0)
 __device__ __forceinline__ int split_exp(float amax) {
-    return amax == 0.f ? 0 : 14 + 127 - (int)(__float_as_uint(amax) >> 23);
+    return min(14 + 127 - (int)(__float_as_uint(amax) >> 23), 126);
 }
 __device__ __forceinline__ float pow2i(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
 
@@ -986,9 +995,10 @@ struct PrefillSpShared {
         float o[kPfSpGroups * kPfSpRows * QS];  // the Q rows, then the groups' O rows
         PrefillKsShared<HD> ks;
     };
-    float am[kPfSpGroups][2][2];  // the next tile's largest |K| and |V| per wave
+    float kx[kPfSpGroups][kPfSpKeys];  // 2^-e of the tile's keys
+    float am[kPfSpGroups][2];          // the next tile's largest |V| per wave
     float mm[kPfSpGroups][kPfSpRows], ll[kPfSpGroups][kPfSpRows];
-    int ve[kPfSpGroups][2];       // each wave's last V exponent
+    int ve[kPfSpGroups][2];            // each wave's last V exponent
     int redo;
 };
 
@@ -1049,23 +1059,15 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
         ko += (uint32_t)(kPfSpKeys * NG) * rowb;
         vo += (uint32_t)(kPfSpKeys * NG) * rowb;
     };
-    // the loaded rows' largest magnitudes, for both waves to agree on the scale
+    // the loaded V rows' largest magnitude, for both waves to agree on the scale
     auto publish_max = [&] {
-        float mk = 0.f, mv = 0.f;
-#pragma unroll
-        for (int s = 0; s < KS; s++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) mk = fmaxf(mk, fabsf(kr[s][e]));
+        float mv = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; e++)
 #pragma unroll
             for (int j = 0; j < VD; j++) mv = fmaxf(mv, fabsf(vr[e][j]));
-        mk = wave_max_bcast(mk);
         mv = wave_max_bcast(mv);
-        if (lane == 0) {
-            sh.am[kg][qb][0] = mk;
-            sh.am[kg][qb][1] = mv;
-        }
+        if (lane == 0) sh.am[kg][qb] = mv;
     };
     if (kg < ntile) load();
 
@@ -1098,30 +1100,24 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
     }
     // B of S^T: query row 32*qb + 16*j + col, the dims of K's operands
     uint4 qp[2][KS][2];
-    bool fine;
-    float c;  // log2(e) / sqrt(HD) over the Q scale
-    {
-        float qv[2][KS][8], mq = 0.f;
+    float c[2];  // log2(e) / sqrt(HD) over the row's scale
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+    for (int j = 0; j < 2; j++) {
+        float qv[KS][8], mq = 0.f;
 #pragma unroll
-            for (int s = 0; s < KS; s++) {
-                const float* p = sh.o + (32 * qb + 16 * j + col) * QS + 32 * s + 4 * grp;
-                const float4 x = *reinterpret_cast<const float4*>(p);
-                const float4 y = *reinterpret_cast<const float4*>(p + 16);
-                qv[j][s][0] = x.x; qv[j][s][1] = x.y; qv[j][s][2] = x.z; qv[j][s][3] = x.w;
-                qv[j][s][4] = y.x; qv[j][s][5] = y.y; qv[j][s][6] = y.z; qv[j][s][7] = y.w;
+        for (int s = 0; s < KS; s++) {
+            const float* p = sh.o + (32 * qb + 16 * j + col) * QS + 32 * s + 4 * grp;
+            const float4 x = *reinterpret_cast<const float4*>(p);
+            const float4 y = *reinterpret_cast<const float4*>(p + 16);
+            qv[s][0] = x.x; qv[s][1] = x.y; qv[s][2] = x.z; qv[s][3] = x.w;
+            qv[s][4] = y.x; qv[s][5] = y.y; qv[s][6] = y.z; qv[s][7] = y.w;
 #pragma unroll
-                for (int e = 0; e < 8; e++) mq = fmaxf(mq, fabsf(qv[j][s][e]));
-            }
-        mq = wave_max_bcast(mq);
-        fine = split_range(mq);
-        const int e = fine ? split_exp(mq) : 0;
+            for (int e = 0; e < 8; e++) mq = fmaxf(mq, fabsf(qv[s][e]));
+        }
+        const int e = split_exp(max_over_groups(mq));
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int s = 0; s < KS; s++) split2x8(qv[j][s], pow2i(e), qp[j][s][0], qp[j][s][1]);
-        c = 1.44269504088896341f / sqrtf((float)HD) * pow2i(-e);
+        for (int s = 0; s < KS; s++) split2x8<1>(qv[s], pow2i(e), qp[j][s][0], qp[j][s][1]);
+        c[j] = 1.44269504088896341f / sqrtf((float)HD) * pow2i(-e);
     }
     int qpos[2];
 #pragma unroll
@@ -1135,7 +1131,7 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
     const bool wave_rows = 32 * qb / G < QT && qt0 + 32 * qb / G < n_tok;
 
     float M[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
-    int ve = 0;  // o is in units of 2^-ve
+    int vs = 126, ve = 126;  // V's scale is 2^vs, the same in both waves; o is in units of 2^-ve
     v4f_t o[2][DT];
 #pragma unroll
     for (int j = 0; j < 2; j++)
@@ -1147,18 +1143,21 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
         const int kt = NG * it + kg;
         if (kt < ntile) publish_max();
         __syncthreads();  // the Q rows, or the last tile's fragments, are read
-        int ke = 0, ven = ve;
         if (kt < ntile) {
-            const float mk = fmaxf(sh.am[kg][0][0], sh.am[kg][1][0]);
-            const float mv = fmaxf(sh.am[kg][0][1], sh.am[kg][1][1]);
-            const bool ok = split_range(mk) && split_range(mv);
-            fine = fine && ok;
-            ke = __builtin_amdgcn_readfirstlane(ok ? split_exp(mk) : 0);
-            ven = __builtin_amdgcn_readfirstlane(ok ? split_exp(mv) : 0);
+            // at most the scale so far: raising it could carry o past fp32
+            const float mv = fmaxf(sh.am[kg][0], sh.am[kg][1]);
+            vs = min(vs, __builtin_amdgcn_readfirstlane(split_exp(mv)));
+            float mk = 0.f;  // of key 16*qb + col
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) mk = fmaxf(mk, fabsf(kr[s][e]));
+            const int ke = split_exp(max_over_groups(mk));
+            if (grp == 0) sh.kx[kg][16 * qb + col] = pow2i(-ke);
 #pragma unroll
             for (int s = 0; s < KS; s++) {
                 uint4 p[2];
-                split2x8(kr[s], pow2i(ke), p[0], p[1]);
+                split2x8<1>(kr[s], pow2i(ke), p[0], p[1]);
 #pragma unroll
                 for (int u = 0; u < 2; u++) sh.k[kg][((qb * KS + s) * 2 + u) * 64 + lane] = p[u];
             }
@@ -1167,7 +1166,7 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
                 const float v[8] = {vr[0][j], vr[1][j], vr[2][j], vr[3][j],
                                     vr[4][j], vr[5][j], vr[6][j], vr[7][j]};
                 uint4 p[2];
-                split2x8(v, pow2i(ven), p[0], p[1]);
+                split2x8<kPfSpLow>(v, pow2i(vs), p[0], p[1]);
 #pragma unroll
                 for (int u = 0; u < 2; u++)
                     sh.v[kg][((VD * (dg & 1) + j) * 2 + u) * 64 + vg * 16 + (dg >> 1)] = p[u];
@@ -1198,9 +1197,14 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
             }
         // online softmax of query col over its 8 keys of this lane
         const bool diag = kPfSpKeys * kt + kPfSpKeys - 1 > wave_lo;
-        const float ck = c * pow2i(-ke);
-        const float dv = pow2i(ven - ve);
-        ve = ven;
+        const float dv = pow2i(max(vs - ve, -126));
+        ve = vs;
+        float kx[8];
+#pragma unroll
+        for (int k2 = 0; k2 < 2; k2++) {
+            const float4 x = *reinterpret_cast<const float4*>(sh.kx[kg] + 16 * k2 + 4 * grp);
+            kx[4 * k2] = x.x; kx[4 * k2 + 1] = x.y; kx[4 * k2 + 2] = x.z; kx[4 * k2 + 3] = x.w;
+        }
         float alpha[2];
         uint4 pp[2][2];
 #pragma unroll
@@ -1208,12 +1212,12 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
             float sv[8], tmax = -INFINITY;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                sv[e] = s[e >> 2][j][e & 3];
+                sv[e] = s[e >> 2][j][e & 3] * kx[e];
                 if (diag && kPfSpKeys * kt + 16 * (e >> 2) + 4 * grp + (e & 3) > qpos[j])
                     sv[e] = -INFINITY;
                 tmax = fmaxf(tmax, sv[e]);
             }
-            const float Mn = fmaxf(M[j], ceilf(max_over_groups(tmax) * ck));
+            const float Mn = fmaxf(M[j], ceilf(max_over_groups(tmax) * c[j]));
             // a row with nothing to attend to yet keeps zero weights
             const float Mr = Mn == -INFINITY ? 0.f : Mn - 14.f;  // p in units of 2^-14
             alpha[j] = Mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(M[j] - Mn);
@@ -1221,12 +1225,22 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
             float ps = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                sv[e] = __builtin_amdgcn_exp2f(fmaf(sv[e], ck, -Mr));
+                sv[e] = __builtin_amdgcn_exp2f(fmaf(sv[e], c[j], -Mr));
                 ps += sv[e];
             }
             l[j] = fmaf(l[j], alpha[j], ps);
             alpha[j] *= dv;
-            split2x8(sv, 1.f, pp[j][0], pp[j][1]);
+            split2x8<kPfSpLow>(sv, 1.f, pp[j][0], pp[j][1]);
+        }
+        // whole exponents change seldom, past the first tiles (rescaling by one fma per
+        // sum took 156 us at the shape above: 34 spilled registers instead of 12)
+        if (__any(alpha[0] != 1.f || alpha[1] != 1.f)) {
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[j][t][r] *= alpha[j];
         }
 #pragma unroll
         for (int t = 0; t < DT; t++) {
@@ -1234,14 +1248,15 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
             const uint4 vh = f[0], vl = f[64];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                v4f_t x = mfma_h(vl, pp[j][0], zero);
-                x = mfma_h(vh, pp[j][1], x);
-                x = mfma_h(vh, pp[j][0], x);
+                v4f_t y = mfma_h(vl, pp[j][0], zero);
+                y = mfma_h(vh, pp[j][1], y);
+                const v4f_t x = mfma_h(vh, pp[j][0], zero);
 #pragma unroll
-                for (int r = 0; r < 4; r++) o[j][t][r] = fmaf(o[j][t][r], alpha[j], x[r]);
+                for (int r = 0; r < 4; r++) o[j][t][r] += fmaf(y[r], 1.f / kPfSpLow, x[r]);
             }
         }
     }
+    bool fine = true;
     // the final M decides: an earlier one far below it left weights of 2^(M_old - M) = 0
 #pragma unroll
     for (int j = 0; j < 2; j++) fine = fine && (M[j] == -INFINITY || fabsf(M[j]) <= kPfSpMaxM);
@@ -1300,10 +1315,12 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < NG; w++) {
-            const float f = sh.mm[w][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sh.mm[w][r] - Mx);
+            // l and o in units of 2^-14 (and 2^-ve): f first, so that o stays in range
+            const float f = sh.mm[w][r] == -INFINITY ? 0.f
+                                                     : __builtin_amdgcn_exp2f(sh.mm[w][r] - Mx - 14.f);
             L = fmaf(sh.ll[w][r], f, L);
-            v = fma4(f * pow2i(-sh.ve[w][r >> 5]),
-                     *reinterpret_cast<const float4*>(sh.o + (w * R + r) * QS + 4 * c4), v);
+            const float4 x = *reinterpret_cast<const float4*>(sh.o + (w * R + r) * QS + 4 * c4);
+            v = fma4(pow2i(-sh.ve[w][r >> 5]), make_float4(x.x * f, x.y * f, x.z * f, x.w * f), v);
         }
         const float inv = L > 0.f ? 1.f / L : 0.f;
         v = make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);

@@ -170,3 +170,57 @@ def test_cache_past_32_bit_offsets(ctx):
             smax = np.linalg.norm(qt) * np.linalg.norm(k, axis=1).max() / np.sqrt(hd)
             tol = ((32 + seen / 64) * 2.0 ** -24 + 2.0 ** -22 * smax) * (w @ np.abs(v))
             assert (np.abs(got[t, h] - w @ v) <= tol).all(), (t, h)
+
+
+@pytest.mark.parametrize("H,KVH", [(32, 32), (64, 16)])
+@pytest.mark.parametrize("kind", ["q rows", "k keys", "v channels", "v keys", "v later key", "qkv"])
+def test_split_products_mixed_magnitudes(ctx, H, KVH, kind):
+    """Rows, keys and channels of very different size next to each other: every output as
+    near to 64 bits as fp32 sums of its own terms, whatever the largest beside them."""
+    hd, T, pos0 = 128, 512, 512
+    n, G = pos0 + T, H // KVH
+    rng = np.random.default_rng(len(kind) + H)
+    q = rng.standard_normal((T, H, hd)).astype(np.float32)
+    kc = rng.standard_normal((n, KVH, hd)).astype(np.float32)
+    vc = rng.standard_normal((n, KVH, hd)).astype(np.float32)
+
+    def powers(lo, hi, *shape):
+        return np.exp2(rng.integers(lo, hi + 1, shape)).astype(np.float32)
+
+    if kind in ("q rows", "qkv"):  # up to scores of 2^16
+        q *= powers(-14, 12, T, H, 1)
+    if kind in ("k keys", "qkv"):
+        kc *= powers(-30, 3, n, KVH, 1)
+    if kind in ("v channels", "qkv"):
+        vc *= powers(-26, 0, 1, KVH, hd)
+    if kind == "v keys":
+        vc *= powers(-13, 13, n, KVH, 1)
+    if kind == "v later key":  # earlier rows of its tile give it no weight
+        vc[700] *= 2.0 ** 24
+        vc[813, :, 1::2] *= 2.0 ** 24
+    q = q.reshape(T, H * hd)
+    cos_t, sin_t = O.rope_table(hd, 10000.0, n)
+    got, _ = attend(ctx, q, kc.ravel(), vc.ravel(), pos0, H, KVH, hd, cos_t, sin_t)
+    got = got.reshape(T, H, hd)
+    worst = 0.0
+    for t in sorted({*range(0, T, 23), 186, 187, 188, 288, 299, 300, 301, 302}):
+        qt = O.rope(q[t], pos0 + t, H, hd, cos_t, sin_t).reshape(H, hd).astype(np.float64)
+        seen = pos0 + t + 1
+        for h in range(t % 3, H, 3):
+            k, v = kc[:seen, h // G].astype(np.float64), vc[:seen, h // G].astype(np.float64)
+            s = k @ qt[h] / np.sqrt(hd)
+            w = np.exp(s - s.max())
+            w /= w.sum()
+            # a score is off by 3 * 2^-22 of sum |q||k| / sqrt(hd) at most (the parts' last
+            # bits 2^-23 each, l * l 2^-22, RoPE and the sums 2^-22), which moves the output
+            # by that much of its weight times |v - out|; the weights and the sum of p v take
+            # a few roundings each
+            out = w @ v
+            ds = 3 * 2.0 ** -22 * (np.abs(k) @ np.abs(qt[h])) / np.sqrt(hd) + 2.0 ** -22 * np.abs(s - s.max())
+            # (the weights and V keep 2^-50 of their largest whatever their size)
+            tol = (w * ds) @ np.abs(v - out) + 48 * 2.0 ** -24 * (w @ np.abs(v))
+            tol += 2.0 ** -50 * (np.abs(v).sum(0) + np.abs(v).max())
+            ratio = float((np.abs(got[t, h] - out) / tol).max())
+            worst = max(worst, ratio)
+            assert ratio <= 1, (t, h, ratio)
+    print(kind, "largest error over its bound:", round(worst, 3))
