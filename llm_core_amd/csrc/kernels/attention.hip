@@ -1336,16 +1336,23 @@ static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
     const int nt = a.n_tok > 1 ? a.n_tok : 1;
     if constexpr (HD <= 128) {
         if constexpr (HD == 128) {
-            // the split products where 64-row workgroups nearly fill the chip and walk
-            // enough keys to pay for setting up (32 heads, 512 tokens, position 0:
-            // 44 us there, 48 here; from about position 300 on this one is faster).
-            // With 128 of them, or at head dimension 64, the 16-row kernel is ahead
-            // (16/2 heads, 512 tokens on 2000 keys: 126 and 166 us).
-            const int QS = kPfSpRows / G;
+            // The split products where their 64-row workgroups (one a CU) nearly fill the
+            // chip in fewer rounds than the 16-row kernel's (three a CU), and from a mean
+            // position of 640 on (40 heads, 320 tokens after 640: 91 us there, 75 here; 32
+            // heads, 512 tokens at position 0: 43 and 48), or in as many rounds from 1024
+            // on (64 heads, 192 tokens after 640 or 2500: 61 and 189 us there, 66 and 171
+            // here).  With few of a workgroup's 64 rows in use, with 128 workgroups or at
+            // head dimension 64 the 16-row kernel is ahead (192 heads, 16 tokens after
+            // 2500: 98 us there, 170 here; 16/2 heads, 512 tokens on 2000 keys: 116 and 166).
+            const int QS = kPfSpRows / G, QT16 = kPfKsRows / G;
             const dim3 gs((unsigned)a.n_kv_heads, (unsigned)((nt + QS - 1) / QS));
+            const long n64 = (long)gs.x * gs.y, n16 = (long)a.n_kv_heads * ((nt + QT16 - 1) / QT16);
+            const long rounds64 = (n64 + 255) / 256, rounds16 = (n16 + 767) / 768;
+            const long mean = a.pos + nt / 2;
             // its K and V row offsets are 32-bit, up to 160 rows past the last key
             const bool offsets = ((uint64_t)a.pos + nt + 160) * a.n_kv_heads * HD * 4 <= UINT32_MAX;
-            if (gs.x * gs.y >= 192 && !a.pos_dev && a.pos + nt / 2 >= 640 && offsets) {
+            if (n64 >= 192 && n16 > 512 && offsets && !a.pos_dev &&
+                (rounds64 < rounds16 ? mean >= 640 : rounds64 == rounds16 && mean >= 1024)) {
                 hipLaunchKernelGGL((k_attn_prefill_sp<HD>), gs, dim3(kPfSpThreads), 0, st, a, G, QS);
                 return hipGetLastError();
             }

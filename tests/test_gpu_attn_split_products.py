@@ -25,9 +25,13 @@ def attend(ctx, q, kc, vc, pos0, H, KVH, hd, cos_t, sin_t, path=0):
 
 
 @pytest.mark.parametrize("H,KVH,T,pos0,kscale,vscale", [
-    (24, 24, 512, 384, 1.0, 1.0),     # exactly 192 workgroups, mean position 640
+    (24, 24, 512, 384, 1.0, 1.0),     # 192 workgroups, as many rounds either way: the 16-row kernel
+    (24, 24, 512, 768, 1.0, 1.0),     # the same, its first mean position (1024)
+    (32, 32, 400, 440, 1.0, 1.0),     # fewer rounds, their first mean position (640)
+    (64, 8, 190, 930, 1.0, 1.0),      # 8 heads per kv head, 8 tokens per workgroup, past 1024
+    (172, 172, 66, 1100, 1.0, 1.0),   # two rounds either way, the second group's rows hardly used
     (28, 4, 440, 500, 1.0, 1.0),      # 7 heads per kv head: 9 tokens (63 rows), the last group ragged
-    (64, 8, 190, 700, 1.0, 1.0),      # 8 heads per kv head, 8 tokens per workgroup
+    (64, 8, 190, 700, 1.0, 1.0),
     (40, 40, 300, 1000, 3e-5, 1e9),   # small K (uniform weights), large V
     (40, 40, 300, 1000, 40.0, 1e-8),  # one key takes nearly all of each row
 ])
