@@ -1265,11 +1265,16 @@ __global__ __launch_bounds__(StageW::NW * 64, 2) void k_gemm_f16_q4k_wide(WideAr
     }
 }
 
-// Where the wide tiles run: from one workgroup per CU on (below, the 32-token
-// groups of k_gemm_f16_q4k leave fewer CUs idle; at exactly 256, 4096 x 4096
-// and 512 tokens, 52.8 -> 51.6 us).
+// Where the wide tiles run: from one workgroup per CU on, and where the CU with
+// the most of them is done sooner than with 128 x 32 tiles of k_gemm_f16_q4k.
+// At 2048 columns, activations' quantisation and re-layout included, k tiles
+// take 10 k + 9.5 us there and 29, 41, 57.5, 73, 87, 101 us here for k = 1 .. 6
+// (214 shapes, 4096 to 32000 rows): 11008 rows, 321 tokens 50.5 (4 tiles) and
+// 57.9 us (3), 512 tokens 71.0 (6) and 59.6 us (3).
 bool wide_applies(int rows, int T) {
-    return T >= 64 && (long)((rows + 127) / 128) * ((T + 63) / 64) >= 256;
+    const long nrt = (rows + 127) / 128, tiles = nrt * ((T + 63) / 64);
+    const long wide = (tiles + 255) / 256, narrow = (nrt * ((T + 31) / 32) + 255) / 256;
+    return T >= 64 && tiles >= 256 && 3 * wide < 2 * narrow;
 }
 
 template <bool SW>
@@ -2019,7 +2024,7 @@ hipError_t launch_gemm_f16_q4k_xh(float* Y, uint8_t* hq8, float* hf, const void*
         (hxh && (Tp % 64 || !hdx2 || !hgx2 || !hdx4)))
         return hipErrorInvalidValue;
     const auto* w = static_cast<const uint8_t*>(W);
-    if (wide_applies(rows, T)) {
+    if (wide_applies(rows, Tp)) {  // the 32-token groups cover the padding here
         if (swiglu)
             launch_wide<true>(nullptr, w, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, 0, hq8, hf,
                               hxh, hdx2, hgx2, hdx4);

@@ -11,11 +11,16 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,cols,T", [
-    (32768, 256, 65),     # 256 x 2 groups, the second of one token (Tp % 64 == 32), one super-block
-    (16385, 512, 97),     # a last row tile of one row, 33 tokens in the last group
+    (8192, 256, 193),     # 4 groups, the last of one token (Tp % 64 == 32), one super-block
+    (8100, 512, 209),     # a ragged last row tile, 17 tokens in the last group
+    (16385, 256, 520),    # 129 row tiles, the last of one row; 5 wide tiles a CU against 9
+    (8191, 512, 385),     # 2 wide tiles a CU against 4
+    (32768, 256, 65),     # as many (2 against 3): the 128 x 32 tiles
+    (16385, 512, 97),
     (8191, 1024, 256),    # rows % 4 != 0: per-row stores
     (4096, 512, 512),     # exactly 256 workgroups
-    (4224, 768, 491),     # 33 row tiles: XCD 0 has one more than the others
+    (4224, 768, 491),     # 2 against 3: the 128 x 32 tiles, 33 of them
+    (8320, 768, 385),     # 65 row tiles: XCD 0 has one more than the others
 ])
 def test_gemm_wide(ctx, rows, cols, T):
     W = hip.synth_weight(12, rows, cols, seed=rows + T)
