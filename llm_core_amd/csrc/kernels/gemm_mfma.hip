@@ -1815,25 +1815,54 @@ __global__ __launch_bounds__(RT * 64) void k_gemm_f16_q6k(
 // two 64 KiB stages)
 constexpr int kF16Q6RT = 8, kF16Q6TTW = 4, kF16Q6S = 2;
 
-// K ranges of the fp16 kernel (a CU holds one workgroup): one from 192 tiles of
-// 128 x 64 up, below that as many as fit 256 workgroups; 0: the int8 kernel's
-// small tiles instead.  Those scale every result on the VALU, but fill the chip
-// by themselves and store no partial sums: ranges pay from 3 super-blocks on,
-// and where 64 x 64 tiles fill the chip already (128 tiles of ours) from 12.
-// With the activations' quantisation and re-layout, int8 -> here: 4096 x 11008
-// at 64 tokens 41.9 -> 38.4 us, at 100 75.9 -> 56.1, 2048 x 11008 at 200
-// 76.1 -> 56.5, 4096 x 11008 at 400 (224 tiles, one range) 197 -> 166.  Below
-// the lines: 4096 x 4096 at 64 tokens (2 super-blocks a range) 18.9 -> 23.0,
-// 4096 x 2048 at 200 (128 tiles, 4) 25.3 -> 29.3.
+// Tile choice: the largest of 64x64, 32x32, 16x16 (rows x tokens) whose grid
+// still has one workgroup per CU; below that the 16x16 tile with the widest
+// K split.  (Measured on 4096 x 11008 and 2048 x 11008 matrices, T = 8..256.)
+enum class Tile6 { R64T64, R32T32, R16T16, R16T16K8 };
+
+Tile6 pick6(int rows, int T) {
+    auto grid = [&](int rw, int tw) {
+        return (long)((rows + rw - 1) / rw) * (long)((T + tw - 1) / tw);
+    };
+    constexpr long kFill = 256;
+    if (T <= 16) return Tile6::R16T16K8;
+    if (grid(64, 64) >= kFill) return Tile6::R64T64;
+    if (grid(32, 32) >= kFill) return Tile6::R32T32;
+    if (grid(16, 16) >= kFill) return Tile6::R16T16;
+    return Tile6::R16T16K8;
+}
+
+int tokens6(Tile6 t) { return t == Tile6::R64T64 ? 64 : (t == Tile6::R32T32 ? 32 : 16); }
+
+// K ranges of the fp16 kernel: as many as leave the fullest XCD one workgroup
+// per CU (row tiles go round the 8 XCDs of 32 CUs, a CU holds one workgroup);
+// 0: the int8 kernel's tiles instead.  Those scale every result on the VALU, but
+// are smaller, fill the chip by themselves and store no partial sums.  Both cost
+// what their fullest CU's work costs, in microseconds over 1632 shapes (256 to
+// 14336 rows, 1024 to 14336 columns, 33 to 512 tokens): 3.45 a super-block and
+// round here, and 6 where partial sums are stored and added; 2.08, 0.72, 0.25
+// and 0.23 a super-block and round of 256 tiles for the int8 kernel's four
+// tiles.  The sooner done is taken, from 3 super-blocks a range (below, filling
+// the pipeline is most of it): 0.2% over the faster of the two on average.
+// int8 -> here, quantisation and re-layout included: 4096 x 11008 at 64 tokens
+// 40.5 -> 36.9 us, at 100 74.8 -> 54.3, at 400 (one range) 197 -> 167, 2560 x
+// 11008 at 300 142 -> 94.  The int8 kernel keeps 2560 x 11008 at 48 tokens (28.9
+// us; 11 ranges, 33 workgroups on half the XCDs, take 42.2), 4096 x 4096 at 64
+// and 512 x 11008 at 512 (47.2; 8 ranges 68.5).
 int q6_ranges(int rows, int T, int nb, int* kper) {
     *kper = nb;
     if (T <= 32) return 0;  // 64-token tiles would be half empty
-    const long tiles = (long)((rows + 127) / 128) * ((T + 63) / 64);
-    if (tiles >= 192) return 1;
-    const int want = (int)(256 / tiles);
-    if (want == 1) return 0;
-    *kper = (nb + want - 1) / want;
-    return *kper >= (tiles >= 128 ? 12 : 3) ? (nb + *kper - 1) / *kper : 0;
+    auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
+    const long per_xcd = cdiv(cdiv(rows, 128), 8) * cdiv(T, 64);
+    if (per_xcd < 32) *kper = (int)cdiv(nb, 32 / per_xcd);
+    const int ranges = (int)cdiv(nb, *kper);
+    const double here = 3.45 * *kper * cdiv(per_xcd * ranges, 32) + (ranges > 1 ? 6 : 0);
+    const Tile6 tile = pick6(rows, T);
+    const int side = tokens6(tile);
+    const double block = tile == Tile6::R64T64 ? 2.08 : tile == Tile6::R32T32 ? 0.72
+                       : tile == Tile6::R16T16 ? 0.25 : 0.23;
+    const double int8 = block * nb * cdiv(cdiv(rows, side) * cdiv(T, side), 256);
+    return here < int8 && (ranges == 1 || *kper >= 3) ? ranges : 0;
 }
 
 // partial sums: at most 256 tiles of 128 x 64
@@ -1890,25 +1919,6 @@ void launch6h(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scratch, 
                            Y, part, m, ranges, accumulate, vec);
     }
 }
-
-// Tile choice: the largest of 64x64, 32x32, 16x16 (rows x tokens) whose grid
-// still has one workgroup per CU; below that the 16x16 tile with the widest
-// K split.  (Measured on 4096 x 11008 and 2048 x 11008 matrices, T = 8..256.)
-enum class Tile6 { R64T64, R32T32, R16T16, R16T16K8 };
-
-Tile6 pick6(int rows, int T) {
-    auto grid = [&](int rw, int tw) {
-        return (long)((rows + rw - 1) / rw) * (long)((T + tw - 1) / tw);
-    };
-    constexpr long kFill = 256;
-    if (T <= 16) return Tile6::R16T16K8;
-    if (grid(64, 64) >= kFill) return Tile6::R64T64;
-    if (grid(32, 32) >= kFill) return Tile6::R32T32;
-    if (grid(16, 16) >= kFill) return Tile6::R16T16;
-    return Tile6::R16T16K8;
-}
-
-int tokens6(Tile6 t) { return t == Tile6::R64T64 ? 64 : (t == Tile6::R32T32 ? 32 : 16); }
 
 struct MfmaCfg {
     int rt, tt;

@@ -45,6 +45,9 @@ def test_gemm_wide(ctx, rows, cols, T):
     (1024, 11008, 65),    # 8 row tiles x 2 groups, 43 super-blocks in 15 ranges
     (2048, 6144, 512),    # 128 tiles: 2 ranges of 12
     (24640, 512, 40),     # 193 tiles, one range
+    (2560, 6144, 129),    # 20 row tiles: three on half the XCDs and two on the others, 3 ranges
+    (4096, 2048, 300),    # 160 tiles, one range
+    (2560, 11008, 48),    # the int8 kernel's 16 x 16 tiles are sooner done
 ])
 def test_gemm_q6k_ranges(ctx, rows, cols, T):
     W = hip.synth_weight(14, rows, cols, seed=rows + T)
