@@ -491,7 +491,8 @@ typedef uint32_t mu4_t __attribute__((ext_vector_type(4)));
 
 // wave tile 16 rows x 64 tokens: the Qwen2.5-0.5B-shape 512-token prefill
 // 6.60 ms against 6.79 (1 x 8 token tiles), 6.76 (2 x 4), 7.17 (2 x 2),
-// 7.32 (1 x 2), 7.83 (4 x 2), 8.98 (2 x 1), 9.59 (4 x 4), 11.0 ms (8 x 2)
+// 7.32 (1 x 2), 7.83 (4 x 2), 8.98 (2 x 1), 9.59 (4 x 4), 11.0 ms (8 x 2);
+// 16 tokens take 16-token wave tiles (Q5_0 896 x 896 10.0 -> 9.1 us)
 constexpr int kMmRTW = 1, kMmTTW = 4, kMmWaves = 4;
 constexpr int kMiscMfmaMinT = 16;  // tokens from which the matrix-core form runs
 
@@ -667,13 +668,13 @@ __device__ __forceinline__ void misc_store(float* __restrict__ Y, const float* _
 // KS waves of a workgroup split K (contiguous block ranges, partial tiles added
 // in wave order through LDS) and kMmWaves / KS waves take consecutive row
 // groups; the block loop loads block b + 1 before computing block b.
-template <int QT, int KS>
+template <int QT, int KS, int TTW>
 __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
     float* __restrict__ Y, const uint8_t* __restrict__ W, const uint8_t* __restrict__ xhl,
     const float* __restrict__ inv, int rows, int cols, long row_bytes, int T, int accumulate) {
-    constexpr int RW = 16 * kMmRTW, TW = 16 * kMmTTW, RG = kMmWaves / KS;
+    constexpr int RW = 16 * kMmRTW, TW = 16 * TTW, RG = kMmWaves / KS;
     static_assert(RG * KS == kMmWaves, "waves");
-    __shared__ mf4_t part[KS > 1 ? KS - 1 : 1][RG][kMmRTW * kMmTTW][64];
+    __shared__ mf4_t part[KS > 1 ? KS - 1 : 1][RG][kMmRTW * TTW][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ks = wave / RG, rg = wave % RG;
@@ -684,28 +685,28 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 #pragma unroll
     for (int i = 0; i < kMmRTW; i++)
         wr[i] = W + min(row0 + 16 * i + col, (long)rows - 1) * row_bytes;  // past the end: not stored
-    const uint8_t* xr[kMmTTW];  // this lane's token: group u = 4b + g's hi at xr + 4b*T*32
+    const uint8_t* xr[TTW];  // this lane's token: group u = 4b + g's hi at xr + 4b*T*32
 #pragma unroll
-    for (int j = 0; j < kMmTTW; j++) {
+    for (int j = 0; j < TTW; j++) {
         const int t = min(t0 + 16 * j + col, T - 1);  // past T: not stored
         xr[j] = xhl + ((size_t)(2 * g) * T + t) * 16;
     }
     const mf4_t zero = {0.f, 0.f, 0.f, 0.f};
-    mf4_t acc[kMmRTW][kMmTTW];
+    mf4_t acc[kMmRTW][TTW];
 #pragma unroll
     for (int i = 0; i < kMmRTW; i++)
 #pragma unroll
-        for (int j = 0; j < kMmTTW; j++) acc[i][j] = zero;
+        for (int j = 0; j < TTW; j++) acc[i][j] = zero;
     const int nb = cols / 32, nbq = (nb + KS - 1) / KS;
     const int b0 = ks * nbq, b1 = min(nb, b0 + nbq);
     MiscRaw raw[kMmRTW];
-    mh8_t xh[kMmTTW], xl[kMmTTW];
+    mh8_t xh[TTW], xl[TTW];
     auto load = [&](int b) {
         const int bb = min(b, nb - 1);  // past the range: a valid block, unused
 #pragma unroll
         for (int i = 0; i < kMmRTW; i++) misc_load<QT>(wr[i], bb, g, raw[i]);
 #pragma unroll
-        for (int j = 0; j < kMmTTW; j++) {
+        for (int j = 0; j < TTW; j++) {
             const uint8_t* p = xr[j] + (size_t)bb * 4 * T * 32;
             xh[j] = *reinterpret_cast<const mh8_t*>(p);
             xl[j] = *reinterpret_cast<const mh8_t*>(p + (size_t)T * 16);
@@ -713,12 +714,12 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
     };
     if (b0 < b1) load(b0);
     for (int b = b0; b < b1; b++) {
-        mh8_t ah[kMmTTW], al[kMmTTW], bw[kMmRTW];
+        mh8_t ah[TTW], al[TTW], bw[kMmRTW];
         float d[kMmRTW];
 #pragma unroll
         for (int i = 0; i < kMmRTW; i++) bw[i] = misc_decode<QT>(raw[i], g, d[i]);
 #pragma unroll
-        for (int j = 0; j < kMmTTW; j++) {
+        for (int j = 0; j < TTW; j++) {
             ah[j] = xh[j];
             al[j] = xl[j];
         }
@@ -726,7 +727,7 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 #pragma unroll
         for (int i = 0; i < kMmRTW; i++)
 #pragma unroll
-            for (int j = 0; j < kMmTTW; j++) {
+            for (int j = 0; j < TTW; j++) {
                 if constexpr (QT == 1) {
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], bw[i], acc[i][j], 0, 0, 0);
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[j], bw[i], acc[i][j], 0, 0, 0);
@@ -744,7 +745,7 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 #pragma unroll
             for (int i = 0; i < kMmRTW; i++)
 #pragma unroll
-                for (int j = 0; j < kMmTTW; j++) part[ks - 1][rg][i * kMmTTW + j][lane] = acc[i][j];
+                for (int j = 0; j < TTW; j++) part[ks - 1][rg][i * TTW + j][lane] = acc[i][j];
         }
         __syncthreads();
         if (ks > 0) return;
@@ -753,11 +754,11 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 #pragma unroll
             for (int i = 0; i < kMmRTW; i++)
 #pragma unroll
-                for (int j = 0; j < kMmTTW; j++) acc[i][j] += part[q][rg][i * kMmTTW + j][lane];
+                for (int j = 0; j < TTW; j++) acc[i][j] += part[q][rg][i * TTW + j][lane];
     }
 #pragma unroll
     for (int i = 0; i < kMmRTW; i++)
-        misc_store<kMmTTW>(Y, inv, acc[i], row0 + 16 * i + col, rows, t0 + 4 * g, T, accumulate);
+        misc_store<TTW>(Y, inv, acc[i], row0 + 16 * i + col, rows, t0 + 4 * g, T, accumulate);
 }
 
 // The same product with a token group's activations shared through LDS: a
@@ -992,19 +993,23 @@ hipError_t launch_gemm_misc_f32(int qtype, float* Y, const void* W, const float*
         }
         // K split over the workgroup's waves where the row groups x token groups
         // leave fewer than 2048 workgroups (K ranges of at least 4 blocks)
-        const long tg = (T + 16 * kMmTTW - 1) / (16 * kMmTTW), nb = cols / 32;
+        const int ttw = T <= 16 ? 1 : kMmTTW;
+        const long tg = (T + 16 * ttw - 1) / (16 * ttw), nb = cols / 32;
         auto wgs = [&](int ks) { return (rows + 16L * kMmRTW * (kMmWaves / ks) - 1) / (16L * kMmRTW * (kMmWaves / ks)) * tg; };
         int ks = 1;
         while (ks < kMmWaves && wgs(ks) < 2048 && nb >= 8L * ks) ks *= 2;
         const dim3 grid((unsigned)(wgs(ks) / tg), (unsigned)tg);
-#define AXF_MM(QT_, KS_) \
-    hipLaunchKernelGGL((k_gemm_misc_mfma<QT_, KS_>), grid, dim3(kMmWaves * 64), 0, st, Y, w8, xhl, iv, rows, cols, row_bytes, T, accumulate)
+#define AXF_MM(QT_, KS_, TTW_) \
+    hipLaunchKernelGGL((k_gemm_misc_mfma<QT_, KS_, TTW_>), grid, dim3(kMmWaves * 64), 0, st, Y, w8, xhl, iv, rows, cols, row_bytes, T, accumulate)
+#define AXF_MM_TTW(QT_, KS_) \
+    do { if (ttw == 1) AXF_MM(QT_, KS_, 1); else AXF_MM(QT_, KS_, kMmTTW); } while (0)
 #define AXF_MM_KS(QT_) \
-    do { if (ks == 4) AXF_MM(QT_, 4); else if (ks == 2) AXF_MM(QT_, 2); else AXF_MM(QT_, 1); } while (0)
+    do { if (ks == 4) AXF_MM_TTW(QT_, 4); else if (ks == 2) AXF_MM_TTW(QT_, 2); else AXF_MM_TTW(QT_, 1); } while (0)
         if (qtype == 1) AXF_MM_KS(1);
         else if (qtype == 8) AXF_MM_KS(8);
         else AXF_MM_KS(6);
 #undef AXF_MM_KS
+#undef AXF_MM_TTW
 #undef AXF_MM
         return hipGetLastError();
     }

@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
     (3072, 928, 250, 0),   # 29 blocks
     (4096, 1024, 192, 0),
     (6144, 96, 128, 2),    # Q5_0 rows that start off a dword keep the general kernel
+    (1000, 1024, 16, 0),   # 16 tokens: the general kernel's 16-token wave tiles, K in 4 ranges,
+    (1000, 288, 16, 0),    # in 2 (the second shorter),
+    (37, 96, 16, 0),       # and whole
 ])
 def test_shared_gemm(ctx, qtype, rows, cols, T, off):
     if off and qtype == AXF_TYPE_F16:
