@@ -1006,7 +1006,8 @@ template <int HD>
 __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, int G, int QT) {
     using SH = PrefillSpShared<HD>;
     constexpr int KS = SH::KS, DT = SH::DT, QS = SH::QS, HALF = HD / 2;
-    constexpr int R = kPfSpRows, NG = kPfSpGroups, VD = HD / 32;  // VD: dims of V per loading lane
+    constexpr int R = kPfSpRows, NG = kPfSpGroups, VD = 4;  // VD: dims of V per loading lane
+    static_assert(HD == 128, "32 lanes load a V row");
     __shared__ SH sh;
 
     const int kvh = blockIdx.x;
@@ -1048,13 +1049,8 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const char* v = vp + min(vo + (uint32_t)(e < 4 ? e : 12 + e) * rowb, lim);
-            if constexpr (VD == 4) {
-                const float4 x = *reinterpret_cast<const float4*>(v);
-                vr[e][0] = x.x; vr[e][1] = x.y; vr[e][2] = x.z; vr[e][3] = x.w;
-            } else {
-                const float2 x = *reinterpret_cast<const float2*>(v);
-                vr[e][0] = x.x; vr[e][1] = x.y;
-            }
+            const float4 x = *reinterpret_cast<const float4*>(v);
+            vr[e][0] = x.x; vr[e][1] = x.y; vr[e][2] = x.z; vr[e][3] = x.w;
         }
         ko += (uint32_t)(kPfSpKeys * NG) * rowb;
         vo += (uint32_t)(kPfSpKeys * NG) * rowb;
@@ -1363,15 +1359,16 @@ static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
         // three, which costs nothing up to one workgroup per CU (32 heads, 33 or 128
         // tokens on 2000 keys: 84 -> 65 us, 91 -> 73 us with them) and more than the
         // prefetch brings from two on (16/2 heads, 512 tokens: 120 -> 126 us)
-        if (HD == 64 || grid.x * grid.y <= 256)
+        const bool prefetch = HD == 64 || grid.x * grid.y <= 256;
+        if (prefetch)
             hipLaunchKernelGGL((k_attn_prefill_ks<HD, true>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
-        else
+        else if constexpr (HD == 128)
             hipLaunchKernelGGL((k_attn_prefill_ks<HD, false>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
-        return hipGetLastError();
+    } else {
+        const int QT = kPfRows / G;
+        const dim3 grid((unsigned)a.n_kv_heads, (unsigned)((nt + QT - 1) / QT));
+        hipLaunchKernelGGL((k_attn_prefill<HD>), grid, dim3(256), 0, st, a, G, QT);
     }
-    const int QT = kPfRows / G;
-    const dim3 grid((unsigned)a.n_kv_heads, (unsigned)((nt + QT - 1) / QT));
-    hipLaunchKernelGGL((k_attn_prefill<HD>), grid, dim3(256), 0, st, a, G, QT);
     return hipGetLastError();
 }
 
