@@ -1270,11 +1270,13 @@ __global__ __launch_bounds__(StageW::NW * 64, 2) void k_gemm_f16_q4k_wide(WideAr
 // At 2048 columns, activations' quantisation and re-layout included, k tiles
 // take 10 k + 9.5 us there and 29, 41, 57.5, 73, 87, 101 us here for k = 1 .. 6
 // (214 shapes, 4096 to 32000 rows): 11008 rows, 321 tokens 50.5 (4 tiles) and
-// 57.9 us (3), 512 tokens 71.0 (6) and 59.6 us (3).
-bool wide_applies(int rows, int T) {
+// 57.9 us (3), 512 tokens 71.0 (6) and 59.6 us (3).  Up to 6 super-blocks 2 tiles
+// here against 3 there, within 2% at longer rows, are the faster too (8960 x 256,
+// 257 tokens 13.9 and 13.2 us).
+bool wide_applies(int rows, int T, int nb) {
     const long nrt = (rows + 127) / 128, tiles = nrt * ((T + 63) / 64);
     const long wide = (tiles + 255) / 256, narrow = (nrt * ((T + 31) / 32) + 255) / 256;
-    return T >= 64 && tiles >= 256 && 3 * wide < 2 * narrow;
+    return T >= 64 && tiles >= 256 && (nb <= 6 ? 3 * wide <= 2 * narrow : 3 * wide < 2 * narrow);
 }
 
 template <bool SW>
@@ -1300,7 +1302,7 @@ void launch16_cfg(float* Y, const uint8_t* W, const uint8_t* XQ8, uint8_t* scrat
     const long n = (long)nkb * Tp;
     hipLaunchKernelGGL(k_gemm_prep16<TTW>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                        XQ8, T, Tp, nkb, xh, dxt, gxt);
-    if (wide_applies(rows, T)) {
+    if (wide_applies(rows, T, nb)) {
         launch_wide<false>(Y, W, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, accumulate);
         return;
     }
@@ -2034,7 +2036,7 @@ hipError_t launch_gemm_f16_q4k_xh(float* Y, uint8_t* hq8, float* hf, const void*
         (hxh && (Tp % 64 || !hdx2 || !hgx2 || !hdx4)))
         return hipErrorInvalidValue;
     const auto* w = static_cast<const uint8_t*>(W);
-    if (wide_applies(rows, Tp)) {  // the 32-token groups cover the padding here
+    if (wide_applies(rows, Tp, nb)) {  // the 32-token groups cover the padding here
         if (swiglu)
             launch_wide<true>(nullptr, w, xh, dxt, gxt, rows, nb, row_bytes, T, Tp, st, 0, hq8, hf,
                               hxh, hdx2, hgx2, hdx4);

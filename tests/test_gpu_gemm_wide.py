@@ -15,12 +15,13 @@ pytestmark = pytest.mark.gpu
     (8100, 512, 209),     # a ragged last row tile, 17 tokens in the last group
     (16385, 256, 520),    # 129 row tiles, the last of one row; 5 wide tiles a CU against 9
     (8191, 512, 385),     # 2 wide tiles a CU against 4
-    (32768, 256, 65),     # as many (2 against 3): the 128 x 32 tiles
+    (32768, 256, 65),     # 2 against 3: wide up to 6 super-blocks,
+    (8200, 1792, 257),    # the 128 x 32 tiles from 7
     (16385, 512, 97),
     (8191, 1024, 256),    # rows % 4 != 0: per-row stores
     (4096, 512, 512),     # exactly 256 workgroups
-    (4224, 768, 491),     # 2 against 3: the 128 x 32 tiles, 33 of them
-    (8320, 768, 385),     # 65 row tiles: XCD 0 has one more than the others
+    (4224, 768, 491),     # 33 row tiles: XCD 0 has one more than the others
+    (8320, 768, 385),     # 65 of them
 ])
 def test_gemm_wide(ctx, rows, cols, T):
     W = hip.synth_weight(12, rows, cols, seed=rows + T)
