@@ -1,6 +1,7 @@
 """The Q8_0 / Q5_0 / F16 GEMM with activations shared through LDS at its edges:
-exactly 192 workgroups, ragged rows and tokens, one block, odd block counts (a
-half-filled last stage, rows that start inside a dword) and W off a dword."""
+exactly 160 workgroups, ragged rows and tokens, one block, odd block counts (a
+half-filled last stage, rows that start inside a dword) and W off a dword; and
+the general kernel just below and at 16 tokens."""
 import numpy as np
 import pytest
 
@@ -13,6 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("qtype", [AXF_TYPE_Q8_0, AXF_TYPE_Q5_0, AXF_TYPE_F16])
 @pytest.mark.parametrize("rows,cols,T,off", [
+    (5120, 256, 128, 0),   # 80 x 2 workgroups, the fewest
+    (5056, 256, 128, 0),   # 79 x 2: the general kernel
     (6144, 32, 100, 0),    # 96 x 2 workgroups, one block: K range 1 is empty
     (6082, 96, 65, 0),     # ragged rows, one token past a group, 3 blocks
     (12226, 160, 33, 0),   # 5 blocks, ragged rows and tokens
