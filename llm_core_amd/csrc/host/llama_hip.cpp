@@ -658,9 +658,11 @@ hipError_t enqueue_step(axf_llama* m, bool device_state, int token, int pos, boo
 //   into the cache; causal attention of every row (q bias and RoPE inside);
 //   o GEMM, x += o; RMSNorm rows -> Q8_0; gate|up GEMM, SwiGLU -> Q8_0;
 //   down GEMM, x += down.
-// Long prompts run as consecutive chunks; every row's arithmetic depends only
-// on its own activations and the cache rows before it, so chunking does not
-// change any result.  After the last chunk: the head of the last row.
+// Long prompts run as consecutive chunks; a row depends only on its own
+// activations and the cache rows before it, but the kernels that run, and with
+// them the order of the fp32 sums, depend on a chunk's tokens and position, so
+// chunking changes results by rounding.  After the last chunk: the head of the
+// last row.
 // ---------------------------------------------------------------------------
 int prefill_alloc(axf_llama* m) {
     if (m->pf_cap) return AXF_OK;

@@ -770,11 +770,12 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 // per row come as 12 (Q5_0) or 20 (Q8_0) dwords, 3 or 5 coalesced loads instead
 // of 14 or 8, spread to the lanes through LDS.  Sums are kept per quarter of K,
 // as with 4 K ranges there.
-// Whole calls before and now, Q5_0 / Q8_0 / F16: 4864 x 896, 512 tokens 49 -> 34,
-// 45 -> 36, 38 -> 29 us; 11008 x 4096, 128 tokens 143 -> 76, 123 -> 98, 93 -> 60 us;
-// 4864 x 896, 200 tokens 28.5 -> 23.9, 26 -> 25, 22 -> 18 us.  Each stage waits for
-// the next one's loads; bringing the first lines into L2 ahead of the loop was
-// slower (25.6 us for 23.9).
+// Whole calls there and here, Q5_0 / Q8_0 / F16: 4864 x 896, 512 tokens 45.5 -> 31.7,
+// 41.9 -> 34.1, 36.5 -> 27.1 us; 11008 x 4096, 128 tokens 143 -> 73, 123 -> 97, 93 -> 59
+// us; 4864 x 896, 200 tokens 25.8 -> 21.6, 24.0 -> 23.9, 21.3 -> 17.6 us.  Each stage
+// waits for the next one's loads (waves wait 40% of their cycles; VALU 28%, matrix
+// cores 11% busy); bringing the first lines into L2 ahead of the loop was 1.7 us
+// slower at the last shape.
 constexpr int kMsWaves = 8, kMsTok = 64, kMsRows = 64;
 
 template <int QT>
@@ -977,8 +978,8 @@ hipError_t launch_gemm_misc_f32(int qtype, float* Y, const void* W, const float*
         const bool dwords = qtype == 1 || (((reinterpret_cast<uintptr_t>(w8) & 3) == 0) &&
                                            ((rows - 1) * row_bytes + cols / 32 * (long)bs) % 4 == 0 &&
                                            row_bytes % 2 == 0);
-        // The shared form from 160 workgroups (2560 x 4096, 200 tokens: Q5_0 79 -> 55 us,
-        // Q8_0 69 -> 61, F16 51 -> 49); with 128 (2048 x 896, 200 tokens) it took 17.1, 17.3
+        // The shared form from 160 workgroups (2560 x 4096, 200 tokens: Q5_0 79 -> 52 us,
+        // Q8_0 68 -> 58, F16 51 -> 45); with 128 (2048 x 896, 200 tokens) it took 17.1, 17.3
         // and 15.1 us against 16.8, 16.2 and 14.6, with fewer it is far behind.  Its offsets
         // are 32-bit.
         if (T > 32 && dwords && (long)gs.x * gs.y >= 160 && (size_t)T * cols * 4 < (1u << 31) &&
