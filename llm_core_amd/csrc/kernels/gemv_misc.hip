@@ -768,8 +768,8 @@ __global__ __launch_bounds__(kMmWaves * 64) void k_gemm_misc_mfma(
 // which bounds it.  Here the four row groups share each 2-block stage (16 KB,
 // loaded into registers during the stage before), and a wave's two blocks
 // per row come as 12 (Q5_0) or 20 (Q8_0) dwords, 3 or 5 coalesced loads instead
-// of 14 or 8, spread to the lanes through LDS.  Sums are kept per quarter of K,
-// as with 4 K ranges there.
+// of 14 or 8, spread to the lanes through LDS.  Sums are kept per quarter of K (of
+// whole pairs of blocks), like the 4 K ranges' there.
 // Whole calls there and here, Q5_0 / Q8_0 / F16: 4864 x 896, 512 tokens 45.5 -> 31.7,
 // 41.9 -> 34.1, 36.5 -> 27.1 us; 11008 x 4096, 128 tokens 143 -> 73, 123 -> 97, 93 -> 59
 // us; 4864 x 896, 200 tokens 25.8 -> 21.6, 24.0 -> 23.9, 21.3 -> 17.6 us.  Each stage
