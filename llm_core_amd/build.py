@@ -71,12 +71,9 @@ def _run(cmd: list[str], cwd: Path | None = None) -> None:
 
 
 # per-source additions: the matrix-core GEMM keeps MFMA results in VGPRs
-# (the default heuristic places them in AGPRs and copies every result out); the
-# prefill attention's key loop starts on an instruction cache line (32 heads of
-# 64, 440 tokens after 300: 34.1 us, and 36.2 us 24 bytes past one)
+# (the default heuristic places them in AGPRs and copies every result out)
 EXTRA_FLAGS = {
     "kernels/gemm_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-    "kernels/attention.hip": ["-falign-loops=64"],
 }
 
 

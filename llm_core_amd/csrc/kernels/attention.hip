@@ -706,7 +706,8 @@ __device__ __forceinline__ void store_out4(const AttnArgs& a, int t, int head, i
 }
 
 // 16 query rows (tokens qt0 .. qt0 + QT - 1) of kv head kvh, one workgroup.
-template <int HD, bool PF>
+// PAD: 4-byte no-ops before the key loop (see launch_prefill_hd).
+template <int HD, bool PF, int PAD>
 __device__ __forceinline__ void prefill_rows16(const AttnArgs& a, int G, int QT, int kvh, int qt0,
                                                PrefillKsShared<HD>& sh) {
     constexpr int KQ = HD / 4;   // dims per lane group: the k-steps of S^T
@@ -795,6 +796,7 @@ __device__ __forceinline__ void prefill_rows16(const AttnArgs& a, int G, int QT,
     };
     // PF: the next tile's rows load during this one
     if (PF && wave < ntile) load(wave);
+    if constexpr (PAD == 1) asm volatile("s_nop 0");
     for (int kt = wave; kt < ntile; kt += NW) {
         float kc[KQ], vc[4][DT];
         if (!PF) load(kt);
@@ -877,11 +879,11 @@ __device__ __forceinline__ void prefill_rows16(const AttnArgs& a, int G, int QT,
     }
 }
 
-template <int HD, bool PF>
+template <int HD, bool PF, int PAD>
 __global__ __launch_bounds__(kPfKsWaves * 64) void k_attn_prefill_ks(AttnArgs a, int G, int QT) {
     __shared__ PrefillKsShared<HD> sh;
     // longest key ranges first
-    prefill_rows16<HD, PF>(a, G, QT, blockIdx.x, (int)(gridDim.y - 1 - blockIdx.y) * QT, sh);
+    prefill_rows16<HD, PF, PAD>(a, G, QT, blockIdx.x, (int)(gridDim.y - 1 - blockIdx.y) * QT, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -1281,7 +1283,7 @@ __global__ __launch_bounds__(kPfSpThreads) void k_attn_prefill_sp(AttnArgs a, in
         const int qt16 = kPfKsRows / G, t_end = min(qt0 + QT, n_tok);
         for (int t = qt0, nt; t < t_end; t += nt) {
             nt = min(qt16 - t % qt16, t_end - t);
-            prefill_rows16<HD, false>(a, G, nt, kvh, t, sh.ks);
+            prefill_rows16<HD, false, 0>(a, G, nt, kvh, t, sh.ks);
             __syncthreads();
         }
         return;
@@ -1361,11 +1363,22 @@ static hipError_t launch_prefill_hd(const AttnArgs& a, int G, hipStream_t st) {
         // three, which costs nothing up to one workgroup per CU (32 heads, 33 or 128
         // tokens on 2000 keys: 84 -> 65 us, 91 -> 73 us with them) and more than the
         // prefetch brings from two on (16/2 heads, 512 tokens: 120 -> 126 us)
-        const bool prefetch = HD == 64 || grid.x * grid.y <= 256;
-        if (prefetch)
-            hipLaunchKernelGGL((k_attn_prefill_ks<HD, true>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
-        else if constexpr (HD == 128)
-            hipLaunchKernelGGL((k_attn_prefill_ks<HD, false>), grid, dim3(kPfKsWaves * 64), 0, st, a, G, QT);
+        const auto block = dim3(kPfKsWaves * 64);
+        if constexpr (HD == 64) {
+            // Where the loop's 8-byte instructions lie counts: up to one round of three
+            // workgroups a CU it is 3-4% the faster with the loop 4 bytes off an 8-byte
+            // boundary (where this build puts it; 32 heads, 200 tokens after 3000: 89.5 us,
+            // 93.1 on one), from two rounds on 6% the faster on one (440 tokens after
+            // 300: 36.2 and 34.1 us; 1 to 15 no-ops before the loop alternate between the two)
+            if ((long)grid.x * grid.y <= 768)
+                hipLaunchKernelGGL((k_attn_prefill_ks<HD, true, 0>), grid, block, 0, st, a, G, QT);
+            else
+                hipLaunchKernelGGL((k_attn_prefill_ks<HD, true, 1>), grid, block, 0, st, a, G, QT);
+        } else if (grid.x * grid.y <= 256) {
+            hipLaunchKernelGGL((k_attn_prefill_ks<HD, true, 0>), grid, block, 0, st, a, G, QT);
+        } else {
+            hipLaunchKernelGGL((k_attn_prefill_ks<HD, false, 0>), grid, block, 0, st, a, G, QT);
+        }
     } else {
         const int QT = kPfRows / G;
         const dim3 grid((unsigned)a.n_kv_heads, (unsigned)((nt + QT - 1) / QT));
